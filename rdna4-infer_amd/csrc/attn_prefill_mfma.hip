@@ -707,32 +707,6 @@ bool prefill_mfma_supported(int kt, int vt, int n_head, int n_head_kv, int head_
   return kt == F16 && vt == F16 && head_dim == kHD && n_head_kv > 0 && n_head % n_head_kv == 0;
 }
 
-// Key splits the MFMA kernel wants for this call: when its row blocks leave
-// CUs idle (the reference engine's 512-query chunks: 64 CTAs on 256 CUs),
-// about one CTA per CU, at most 16 and at most one per key block.
-// RD4_PREFILL_KSPLIT forces a count (1: never split).
-int prefill_ksplits(const PrefillArgs &p) {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      return 0;
-    return n;
-  }();
-  static const int env = [] {
-    const char *e = std::getenv("RD4_PREFILL_KSPLIT");
-    return e ? std::atoi(e) : 0;
-  }();
-  const int grp = p.n_head / p.n_head_kv;
-  const int total = (p.n_q * grp + 191) / 192 * p.n_head_kv;  // the default 192-row CTAs
-  const int max_blocks = (p.kmax + kBN) / kBN;
-  int s = env > 0 ? env : (total % 8 == 0 && 2 * total <= cus) ? cus / total : 1;
-  return std::max(1, std::min(s, std::min(max_blocks, 16)));
-}
-int64_t prefill_part_floats(const PrefillArgs &p, int splits) {
-  return (int64_t)splits * p.n_q * p.n_head * (kHD + 2);
-}
-
 hipError_t prefill_mfma_launch(const PrefillArgs &p, hipStream_t st) {
   static const int shape = [] {
     const char *e = std::getenv("RD4_PREFILL_SHAPE");
@@ -742,18 +716,8 @@ hipError_t prefill_mfma_launch(const PrefillArgs &p, hipStream_t st) {
   const int bm = shape == 2 ? 256 : shape == 0 ? 192 : 128;  // rows per CTA
   const int n_rb = (p.n_q * grp + bm - 1) / bm;
   const int total = n_rb * p.n_head_kv;
-  // Key splits when the row blocks alone leave CUs idle (the reference
-  // engine's 512-query chunks: 64 CTAs on 256 CUs): enough splits of equal
-  // block counts to give about one CTA per CU, if the records fit the scratch.
   PrefillArgs q = p;
-  q.n_ksplit = 1;
-  q.ksplit_blocks = 0;
-  const int s = prefill_ksplits(p);
-  if (s > 1 && p.part && prefill_part_floats(p, s) <= p.part_floats) {
-    const int max_blocks = (p.kmax + kBN) / kBN;
-    q.ksplit_blocks = (max_blocks + s - 1) / s;
-    q.n_ksplit = (max_blocks + q.ksplit_blocks - 1) / q.ksplit_blocks;
-  }
+  prefill_set_ksplits(q, prefill_ksplits(p, F16, F16, p.part_floats), kBN);
   dim3 grid((unsigned)(total * q.n_ksplit));
   if (shape == 1)  // 4 waves x 32 rows (one wave per SIMD)
     hipLaunchKernelGGL((prefill_mfma_kernel<4, 2>), grid, dim3(256), (size_t)kLdsBytes, st, q);
@@ -763,12 +727,14 @@ hipError_t prefill_mfma_launch(const PrefillArgs &p, hipStream_t st) {
     hipLaunchKernelGGL((prefill_mfma_kernel<8, 1>), grid, dim3(512), (size_t)kLdsBytes, st, q);
   else  // 12 waves x 16 rows (three waves per SIMD)
     hipLaunchKernelGGL((prefill_mfma_kernel<12, 1>), grid, dim3(768), (size_t)kLdsBytes, st, q);
-  if (q.n_ksplit > 1) {
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const int64_t rows = (int64_t)p.n_q * p.n_head;
-    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, q);
-  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || q.n_ksplit == 1) return e;
+  return prefill_merge_launch(q, st);
+}
+
+hipError_t prefill_merge_launch(const PrefillArgs &q, hipStream_t st) {
+  const int64_t rows = (int64_t)q.n_q * q.n_head;
+  hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, q);
   return hipGetLastError();
 }
 

@@ -1,0 +1,669 @@
+// Causal GQA prefill over quantized K/V caches (gfx950), head_dim 256: every
+// pair of f16, q8_0, q4_0, q5_0 and q4_1 except f16/f16 (attn_prefill_mfma.hip).
+//
+// Reference semantics: the batched path of graph.cuh:1473-1535 over a quantized
+// cache (attn_split_batch_launch, include/rdna4/attn.cuh:958-1049): query token
+// i at position p_i attends keys 0..min(p_i, kmax), dequantized as kv_load<>
+// (kv.h:174-368), f32 softmax and accumulation, then the optional sigmoid gate.
+//
+// Precision: 32-bit, on f16 matrix instructions. Every operand enters as an
+// f16 hi part plus the f16 remainder:
+//   * a query row is scaled by a power of two (its largest |q * scale * log2e|
+//     comes to [2^8, 2^9)) and split, q' = qh + ql to 2^-22 of the row's largest;
+//   * a quantized key row is scaled by a power of two (its largest block scale
+//     comes to [1, 2)) and split: d * int has at most 19 significant bits, so
+//     K' = kh + kl exactly (blocks down to 2^-14 of the row's largest scale);
+//   * S = kl.qh + kh.ql + kh.qh, f32 accumulation, then times both powers of two;
+//   * p stays f32 for the row sum l; p * 2^(e - e0 + 7) (e the V row's power of
+//     two, e0 that of the CTA's first row) is split for O += vl.ph + vh.pl + vh.ph.
+//     The reference exponent of a row follows its largest s + e - e0, so the split
+//     value stays within 2^15 whatever the cache holds.
+// f16 rows have no remainder part (and no scaling): two products instead of three.
+// Relative error against 64 bits, the VALU kernel (attn_generic.hip), which took
+// these calls before, in brackets, for q8_0: 1.2e-7 (1.3e-7) at 33 queries over 33
+// keys, 2.2e-7 (2.9e-7) over 233, 3.5e-7 (9.0e-7) over 8064. What it takes: the
+// large products of S in four sums and the small ones in a fifth (one sum for
+// all: 2.0 times the error at 233 keys), the p split near 2^7 (near 1: 1.5 times),
+// and exp2 arguments near 0 for the largest p (e folded into them: 1.3 times).
+//
+// Work decomposition: rows r = query * group + head of one kv head as in the
+// f16 kernel; CTA = 8 waves x 16 rows, 32-key blocks. Each wave owns 8 key rows of
+// a block (waves 0-3 K, 4-7 V): it brings their raw cache bytes to its own LDS
+// area by DMA two blocks ahead, and a block ahead converts them, 8 lanes per row
+// and one 32-value block per lane, into the hi / lo stage that all waves read.
+// Two stages, one CTA barrier per block. Waves w and w + 4 share a SIMD:
+// waves 0-3 convert before their products, 4-7 after, so that one's conversion
+// runs beside the other's matrix instructions.
+// What bounds it: LDS reads (64 KiB per wave and block, 0.5 MiB per CTA) and the
+// matrix pipe, which takes three products where f16 takes one. 512 queries over
+// 8192 q8_0 keys, 24 / 4 heads: 6120 us in the VALU kernel, 389 us here (0.26
+// PFLOP/s, 0.78 of them counted as issued).
+#include <algorithm>
+#include <cstdlib>
+
+#include "kv_quant.hpp"
+#include "prefill.hpp"
+
+namespace rd4 {
+
+namespace {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef short short4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) short4v lds_short4;
+typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
+
+constexpr int kHD = 256;
+constexpr int kBN = 32;            // keys per block
+constexpr int kW = 8;              // waves per CTA
+constexpr int kBM = 16 * kW;       // rows per CTA
+constexpr int kPart = kBN * kHD * 2;  // one f16 part of a block's K or V rows
+constexpr float kLog2e = 1.4426950408889634f;
+// the largest p * 2^(e - e0) of a row is kept between 2^kPShift and 2^(kPShift + 8):
+// terms 2^-14 of it still have normal f16 remainder parts
+constexpr int kPShift = 7;
+
+// LDS: two stages of [K hi][K lo][V hi][V lo] (lo parts of quantized types
+// only), each wave's raw rows, then the per-key tables of both stages.
+template <bool KLO, bool VLO>
+struct Lds {
+  static constexpr int KH = 0, KL = kPart, VH = (1 + KLO) * kPart, VL = VH + kPart;
+  static constexpr int kStage = (2 + KLO + VLO) * kPart;
+  // 8 rows of a wave in whole 1 KiB DMA instructions: f16 4096 B, else at most 3072
+  static constexpr int kRawK = KLO ? 3072 : 4096, kRawV = VLO ? 3072 : 4096;
+  static constexpr int kRaw = 2 * kStage;
+  static constexpr int kTab = kRaw + 4 * (kRawK + kRawV);
+  // per stage: f32 2^e of K rows, f32 2^(e - e0 + kPShift) and e - e0 of V rows,
+  // and one byte per V row with a bit for each of its blocks that is not finite
+  static constexpr int kTabStage = 3 * kBN * 4 + kBN;
+  static constexpr int kBytes = kTab + 2 * kTabStage;
+  static_assert(kBytes <= 160 * 1024, "LDS of a CU");
+};
+
+// LDS swizzle of a 512-byte f16 row: 16-byte chunk c of key r sits in slot
+// c ^ swz(r) (the f16 prefill kernel's map, conflict-free for the b128 operand
+// reads and for the transposing reads).
+__device__ __forceinline__ int swz(int r) {
+  return ((r & 1) ? 8 : 0) ^ ((r & 2) ? 7 : 0) ^ ((r & 4) ? 2 : 0) ^ ((r & 8) ? 4 : 0);
+}
+
+__device__ __forceinline__ half2v as_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+__device__ __forceinline__ uint32_t as_u32(half2v v) { return __builtin_bit_cast(uint32_t, v); }
+
+// max over lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float max_groups4(float x) {
+  float a = x, b = x;
+  __asm__("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  float c = fmaxf(a, b), d = c;
+  __asm__("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
+  return fmaxf(c, d);
+}
+// unsigned max over the 8 lanes 8k .. 8k + 7
+__device__ __forceinline__ uint32_t max8_u32(uint32_t x) {
+  int v = (int)x;
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));  // row_half_mirror
+  return (uint32_t)v;
+}
+
+// 16 bytes per lane from sbase + voff into LDS at lds + 16 * lane (asm, so the
+// compiler puts no wait for it in front of other LDS reads; the kernel waits)
+__device__ __forceinline__ void dma16(const uint8_t *sbase, uint32_t voff, uint32_t lds) {
+  __asm__ volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                   :
+                   : "v"(voff), "s"(sbase), "s"(lds)
+                   : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t lds_addr(const uint8_t *p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p);
+}
+__device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *ptr) {
+  const uint64_t a = (uint64_t)ptr;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return (const uint8_t *)(((uint64_t)hi << 32) | lo);
+}
+
+// Two integers as an f16 pair times the block scale -> hi pair and exact
+// remainder pair (an f16 product's rounding error is itself an f16).
+__device__ __forceinline__ void split_mul(half2v q, half2v d, uint32_t &hi, uint32_t &lo) {
+  const half2v h = q * d;
+  hi = as_u32(h);
+  lo = as_u32(__builtin_elementwise_fma(q, d, -h));
+}
+// The same with q4_1's offset: d * q + m, the sum's rounding error recovered by
+// a two-sum.
+__device__ __forceinline__ void split_mul_add(half2v q, half2v d, half2v m, uint32_t &hi, uint32_t &lo) {
+  const half2v h = q * d, l = __builtin_elementwise_fma(q, d, -h);
+  const half2v s = h + m, bb = s - h;
+  const half2v err = (h - (s - bb)) + (m - bb);
+  hi = as_u32(s);
+  lo = as_u32(err + l);
+}
+
+// Convert one 32-value block of type T, its bytes in LDS at row + b * block
+// bytes (row 4-byte aligned; blocks start 2 bytes off a word where b is odd
+// except q4_1's), into 16 hi words and 16 lo words (f16 pairs of consecutive
+// elements). pw2 is the power of two that the row's values are scaled by.
+template <int T>
+__device__ __forceinline__ void block_words(const uint8_t *row, int b, uint32_t *w, uint32_t *dm) {
+  // w: the block's data words after d (q5_0: the high bits, then the nibbles; q4_1: nibbles), dm: d | m << 16
+  constexpr int BB = block_bytes(T);
+  constexpr int NW = T == Q8_0 ? 8 : T == Q5_0 ? 5 : 4;
+  const uint32_t *p = (const uint32_t *)(row + ((BB * b) & ~3));
+  if constexpr (T == Q4_1) {
+    *dm = p[0];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) w[i] = p[i + 1];
+  } else {
+    uint32_t x[NW + 1];
+#pragma unroll
+    for (int i = 0; i <= NW; ++i) x[i] = p[i];
+    const bool odd = b & 1;
+    *dm = odd ? x[0] >> 16 : x[0] & 0xffffu;
+    // even blocks: data starts 2 bytes into x[0]; odd blocks: at x[1]
+    const uint32_t sel = odd ? 0x07060504u : 0x05040302u;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) w[i] = __builtin_amdgcn_perm(x[i + 1], x[i], sel);
+  }
+}
+
+template <int T>
+__device__ __forceinline__ void convert_words(const uint32_t *w, half2v d, half2v m, uint32_t hi[16], uint32_t lo[16]) {
+  if constexpr (T == Q8_0) {
+    // f16 1024 + 128 + byte, less 1152 (exact)
+    const half2v c = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      split_mul(as_h2(__builtin_amdgcn_perm(0u, w[i], 0x0c010c00u) ^ 0x64806480u) + c, d, hi[2 * i], lo[2 * i]);
+      split_mul(as_h2(__builtin_amdgcn_perm(0u, w[i], 0x0c030c02u) ^ 0x64806480u) + c, d, hi[2 * i + 1], lo[2 * i + 1]);
+    }
+  } else {
+    constexpr int W0 = T == Q5_0 ? 1 : 0;
+    constexpr float kBias = T == Q4_0 ? -1032.0f : T == Q5_0 ? -1040.0f : -1024.0f;
+    const half2v c = {(_Float16)kBias, (_Float16)kBias};
+#pragma unroll
+    for (int half = 0; half < 2; ++half)  // low nibbles: elements 0..15, high: 16..31
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {       // elements 16 half + 2i, 2i + 1: bytes 2i, 2i + 1
+        const uint32_t by = __builtin_amdgcn_perm(0u, w[W0 + (i >> 1)], (i & 1) ? 0x0c030c02u : 0x0c010c00u);
+        uint32_t n = (half ? by >> 4 : by) & 0x000f000fu;
+        if constexpr (T == Q5_0) {
+          const uint32_t hb = w[0] >> (16 * half + 2 * i);  // bits of the two elements
+          n |= ((hb & 1u) << 4) | ((hb & 2u) << 19);
+        }
+        const half2v q = as_h2(n | 0x64006400u) + c;
+        if constexpr (T == Q4_1) split_mul_add(q, d, m, hi[8 * half + i], lo[8 * half + i]);
+        else split_mul(q, d, hi[8 * half + i], lo[8 * half + i]);
+      }
+  }
+}
+
+// Exponent of a row's power of two, from the f16 magnitude bits of its blocks'
+// scales (one per lane of the row's 8; the largest finite one counts).
+__device__ __forceinline__ int row_exponent(uint32_t mag) {
+  return max((int)(max8_u32(mag >= 0x7c00u ? 0u : mag) >> 10), 1) - 15;
+}
+
+// Convert the wave's 8 raw rows (lane = 8 * row + block) to the hi / lo stage.
+template <int T>
+__device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int lane, uint8_t *hi_st, uint8_t *lo_st,
+                                             float *pw2_tab, float *exp_tab, uint8_t *nf_tab, int e0) {
+  const int r = lane >> 3, b = lane & 7, key = key0 + r;
+  const int dst = key * (kHD * 2), sz = swz(key & 15);
+  if constexpr (T == F16) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *(u32x4 *)(hi_st + dst + 16 * ((4 * b + i) ^ sz)) = *(const u32x4 *)(raw + r * 512 + 64 * b + 16 * i);
+  } else {
+    uint32_t w[8], dm, hi[16], lo[16];
+    block_words<T>(raw + r * (8 * block_bytes(T)), b, w, &dm);
+    // The row's power of two from its largest scale (q4_1: or offset) magnitude.
+    uint32_t mag = dm & 0x7fffu;
+    if (T == Q4_1) mag = max(mag, (dm >> 16) & 0x7fffu);
+    const bool nonfin = mag >= 0x7c00u;
+    const int e = row_exponent(mag);
+    _Float16 d = __builtin_amdgcn_ldexph(__builtin_bit_cast(_Float16, (uint16_t)dm), -e);
+    _Float16 m = T == Q4_1 ? __builtin_amdgcn_ldexph(__builtin_bit_cast(_Float16, (uint16_t)(dm >> 16)), -e) : (_Float16)0.0f;
+    // A block that is not finite: K keeps it (its keys' scores become NaN). V's
+    // enters the products as zeros, so that rows which do not attend the key keep
+    // their sums; nf_tab marks it, and the rows that attend the key end as NaN.
+    if (exp_tab && nonfin) d = (_Float16)0.0f, m = (_Float16)0.0f;
+    convert_words<T>(w, half2v{d, d}, half2v{m, m}, hi, lo);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int off = dst + 16 * ((4 * b + i) ^ sz);
+      *(u32x4 *)(hi_st + off) = u32x4{hi[4 * i], hi[4 * i + 1], hi[4 * i + 2], hi[4 * i + 3]};
+      *(u32x4 *)(lo_st + off) = u32x4{lo[4 * i], lo[4 * i + 1], lo[4 * i + 2], lo[4 * i + 3]};
+    }
+    if (exp_tab) {
+      const uint64_t nf = __ballot(nonfin);
+      if (b == 0) {
+        pw2_tab[key] = __builtin_ldexpf(1.0f, e - e0 + kPShift);
+        exp_tab[key] = (float)(e - e0);
+        nf_tab[key] = (uint8_t)(nf >> (8 * r));
+      }
+    } else if (b == 0) {
+      pw2_tab[key] = __builtin_ldexpf(1.0f, e);
+    }
+  }
+}
+
+}  // namespace
+
+// The kernel's lambdas are its own text: outlined, they put what they capture in scratch.
+#define RD4_INLINE __attribute__((always_inline))
+
+// K fragments and V operand pairs in registers or in flight ahead of their products
+#ifndef RD4_PQ_KD
+#define RD4_PQ_KD 3
+#endif
+#ifndef RD4_PQ_VD
+#define RD4_PQ_VD 3
+#endif
+
+// KLO, VLO: the rows have remainder parts (all but f16); VFULL: q4_1 values, whose
+// remainders are as full as p's, take the fourth product vl.pl too (at 120 queries
+// over 120 keys the error is 1.04 times the VALU kernel's without it, 0.88 with).
+template <bool KLO, bool VLO, bool VFULL>
+__global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p) {
+  using L = Lds<KLO, VLO>;
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int n = lane & 15, g = lane >> 4;
+  const int grp = p.n_head / p.n_head_kv;
+  const int n_rows = p.n_q * grp;
+  const int n_rb = (n_rows + kBM - 1) / kBM;
+  const int total = n_rb * p.n_head_kv;
+  const int ksp = p.n_ksplit > 1 ? (int)blockIdx.x / total : 0;
+  const int Lb = (int)blockIdx.x - ksp * total;
+  // as in the f16 kernel: a kv head's row blocks share the XCDs (and L2s) of that head
+  int kvh, rbp;
+  if (8 % p.n_head_kv == 0 && total % 8 == 0) {
+    const int X = 8 / p.n_head_kv, xcd = Lb % 8, j = Lb / 8;
+    kvh = xcd % p.n_head_kv;
+    rbp = j * X + xcd / p.n_head_kv;
+  } else {
+    kvh = Lb / n_rb;
+    rbp = Lb - kvh * n_rb;
+  }
+  const int r0 = (n_rb - 1 - rbp) * kBM;  // heaviest (latest queries) first
+
+  auto limit_of = [&](int row) RD4_INLINE -> int {
+    if (row >= n_rows) return -1;
+    const int q = row / grp;
+    return min(p.pos ? p.pos[q] : p.pos0 + q, p.kmax);
+  };
+  int kend;  // last key that any row of the CTA attends
+  {
+    int lim = max(limit_of(r0 + lane), limit_of(r0 + 64 + lane));
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) lim = max(lim, __shfl_xor(lim, m, 64));
+    kend = __builtin_amdgcn_readfirstlane(lim);
+  }
+  const int n_blocks = (kend + kBN) / kBN;
+  const int b0 = p.n_ksplit > 1 ? ksp * p.ksplit_blocks : 0;
+  const int nbk = p.n_ksplit > 1 ? max(0, min(n_blocks, b0 + p.ksplit_blocks) - b0) : n_blocks;
+
+  // ---- raw rows of this wave: 8 consecutive keys of each block, K (waves 0-3) or V
+  const bool isv = w >= 4;
+  const int my_t = isv ? p.vt : p.kt;
+  const int rb = __builtin_amdgcn_readfirstlane((int)row_bytes(my_t, kHD)), nch = rb >> 4;
+  const int n_dma = (8 * nch + 63) >> 6;
+  const uint8_t *my_base = (isv ? p.v : p.k) + (int64_t)kvh * rb;
+  const int my_stride = p.n_head_kv * rb;
+  uint8_t *raw = smem + L::kRaw + (isv ? 4 * L::kRawK + (w - 4) * L::kRawV : w * L::kRawK);
+  int c_key[4], c_off[4];  // key in the block and byte in its row of each 16-byte chunk
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int c = min(64 * i + lane, 8 * nch - 1);  // (surplus lanes repeat the last chunk into the padding)
+    c_key[i] = 8 * (w & 3) + c / nch;
+    c_off[i] = 16 * (c % nch);
+  }
+  auto issue = [&](int bi) RD4_INLINE {
+    const int j0 = (b0 + bi) * kBN;
+    const uint8_t *src = uniform_ptr(my_base + (int64_t)j0 * my_stride);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)  // keys past kend re-read a valid row (masked later)
+      if (i < n_dma) dma16(src, (uint32_t)(min(c_key[i], kend - j0) * my_stride + c_off[i]), lds_addr(raw + 1024 * i));
+  };
+  // O and p * 2^e are kept relative to the exponent of the CTA's first V row, so
+  // that p itself is near 1 where it matters (the argument of its exp2 near 0)
+  int e0 = 0;
+  if (VLO && nbk > 0) {
+    const int vrb = (int)row_bytes(p.vt, kHD);
+    const uint8_t *blk = p.v + ((int64_t)b0 * kBN * p.n_head_kv + kvh) * vrb + (lane & 7) * (vrb >> 3);
+    uint32_t mag = ld_u16(blk) & 0x7fffu;
+    if (p.vt == Q4_1) mag = max(mag, (uint32_t)ld_u16(blk + 2) & 0x7fffu);
+    e0 = __builtin_amdgcn_readfirstlane(row_exponent(mag));
+  }
+  auto tab = [&](int st) RD4_INLINE { return (float *)(smem + L::kTab + st * L::kTabStage); };
+  auto convert = [&](int st) RD4_INLINE {
+    uint8_t *sb = smem + st * L::kStage;
+    float *t = tab(st);
+    const int key0 = 8 * (w & 3);
+    if (!isv) {
+      if constexpr (!KLO) convert_rows<F16>(raw, key0, lane, sb + L::KH, nullptr, t, nullptr, nullptr, 0);
+      else switch (p.kt) {
+        case Q8_0: convert_rows<Q8_0>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
+        case Q4_0: convert_rows<Q4_0>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
+        case Q5_0: convert_rows<Q5_0>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
+        default: convert_rows<Q4_1>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
+      }
+    } else {
+      float *vp = t + kBN, *ve = t + 2 * kBN;
+      uint8_t *nf = (uint8_t *)(t + 3 * kBN);
+      if constexpr (!VLO) convert_rows<F16>(raw, key0, lane, sb + L::VH, nullptr, vp, ve, nf, e0);
+      else switch (p.vt) {
+        case Q8_0: convert_rows<Q8_0>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
+        case Q4_0: convert_rows<Q4_0>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
+        case Q5_0: convert_rows<Q5_0>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
+        default: convert_rows<Q4_1>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
+      }
+    }
+  };
+  if (nbk > 0) issue(0);
+
+  // ---- this wave's query rows (row n of the wave is r0 + 16 w + n): scaled, split
+  const int row = r0 + 16 * w + n;
+  const int lim_row = limit_of(row);
+  half8 qh[8], ql[8];
+  float c_row;  // 2^-k: the power of two taken out of the row
+  {
+    const bool on = row < n_rows;
+    const int q = on ? row / grp : 0, head = kvh * grp + (on ? row % grp : 0);
+    const int64_t qoff = ((int64_t)q * p.n_head + head) * kHD + 8 * g;
+    const float sl2 = on ? p.scale * kLog2e : 0.0f;
+    float x[8][8];
+    if (p.q_f16) {
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const half8 h = *(const half8 *)((const uint16_t *)p.q + qoff + 32 * b);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[b][i] = (float)h[i];
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const floatx4 u = *(const floatx4 *)((const float *)p.q + qoff + 32 * b);
+        const floatx4 v = *(const floatx4 *)((const float *)p.q + qoff + 32 * b + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[b][i] = u[i], x[b][4 + i] = v[i];
+      }
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[b][i] *= sl2;
+        mx = fmaxf(mx, fabsf(x[b][i]));
+      }
+    mx = max_groups4(mx);
+    // exponent that brings mx to [2^8, 2^9); zero rows and infinities stay as they are
+    const int ex = (int)(__builtin_bit_cast(uint32_t, mx) >> 23) - 127;
+    const int k = (mx > 0.0f && ex < 128) ? max(-100, min(100, 8 - ex)) : 0;
+    c_row = __builtin_ldexpf(1.0f, -k);
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float y = __builtin_ldexpf(x[b][i], k);
+        const _Float16 h = (_Float16)y;
+        qh[b][i] = h;
+        ql[b][i] = (_Float16)(y - (float)h);
+      }
+  }
+  int wave_min_lim = lim_row;  // blocks whose last key is <= it need no mask
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) wave_min_lim = min(wave_min_lim, __shfl_xor(wave_min_lim, m, 64));
+
+  floatx4 o[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.0f;
+  uint32_t poison = 0;  // 32-dim blocks of this row that met a V block which is not finite
+
+  // transposing V reads (as in the f16 kernel): source lane s of a 16-lane group
+  // points at key 4g + s/4, dims 4(s%4)..+3 of a 16-dim tile
+  const int tr_kx = 4 * g + (n >> 2);
+  const int tr_off = tr_kx * (kHD * 2) + 8 * (n & 1);
+  const int tr_m = 16 * ((n >> 1 & 1) ^ swz(tr_kx));
+  int v_loff[8], k_loff[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    v_loff[i] = tr_off + ((32 * i) ^ tr_m);
+    k_loff[i] = n * (kHD * 2) + 16 * ((4 * i + g) ^ swz(n));
+  }
+
+  // the first block's rows: converted before the loop
+  if (nbk > 0) {
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    convert(0);
+    if (nbk > 1) issue(1);
+  }
+
+  for (int bi = 0; bi < nbk; ++bi) {
+    const int st = bi & 1;
+    const int j0 = (b0 + bi) * kBN;
+    // this wave's raw rows of block bi + 1 have landed, and its conversion of
+    // block bi is written; past the barrier so is every wave's, and all are done
+    // reading the other stage
+    __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    auto next = [&]() RD4_INLINE {
+      if (bi + 1 < nbk) {
+        convert(st ^ 1);
+        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // raw rows read before they are overwritten
+        if (bi + 2 < nbk) issue(bi + 2);
+      }
+    };
+    if (!isv) next();
+    const uint8_t *kd = smem + st * L::kStage + L::KH;
+    const uint8_t *vd = smem + st * L::kStage + L::VH;
+    const float *tb = tab(st);
+
+    // ---- S^T of the two 16-key tiles: fragment f = (dim block f / 2, tile f % 2)
+    // (the small products in a sum of their own and the large ones in four, so that
+    // few roundings happen at the size of the whole sum)
+    floatx4 sc[2][5], s[2];
+#pragma unroll
+    for (int i = 0; i < 10; ++i) sc[i / 5][i % 5] = floatx4{0.f, 0.f, 0.f, 0.f};
+    {
+      constexpr int D = RD4_PQ_KD;
+      u32x4 fh[D], fl[D];
+      auto read_k = [&](int f) RD4_INLINE {
+        const uint8_t *a = kd + (f & 1) * 16 * (kHD * 2) + k_loff[f >> 1];
+        fh[f % D] = *(const lds_u32x4 *)a;
+        if (KLO) fl[f % D] = *(const lds_u32x4 *)(a + kPart);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll
+      for (int f = 0; f < D - 1; ++f) read_k(f);
+#pragma unroll
+      for (int f = 0; f < 16; ++f) {
+        if (f + D - 1 < 16) read_k(f + D - 1);
+        const int b = f >> 1, kt = f & 1;
+        const half8 kh = __builtin_bit_cast(half8, fh[f % D]);
+        floatx4 &sl = sc[kt][4];
+        if (KLO) sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, fl[f % D]), qh[b], sl, 0, 0, 0);
+        sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[b], sl, 0, 0, 0);
+        sc[kt][b & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[b], sc[kt][b & 3], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) s[kt] = ((sc[kt][0] + sc[kt][1]) + (sc[kt][2] + sc[kt][3])) + sc[kt][4];
+
+    // ---- online softmax: lane = row n, keys 16 kt + 4 g + i. The running max
+    // (m_run, in log2) follows s + e (e: the V row's exponent), which bounds p * 2^e.
+    half8 ph, pl;
+    float pf[2][4];
+    {
+      floatx4 vp[2], ve[2];
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        if (KLO) {
+          const floatx4 ks = *(const floatx4 *)(tb + 16 * kt + 4 * g);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[kt][i] *= ks[i];
+        }
+        if (VLO) {
+          vp[kt] = *(const floatx4 *)(tb + kBN + 16 * kt + 4 * g);
+          ve[kt] = *(const floatx4 *)(tb + 2 * kBN + 16 * kt + 4 * g);
+        }
+      }
+      if (j0 + kBN - 1 > wave_min_lim) {  // wave-uniform
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (j0 + 16 * kt + 4 * g + i > lim_row) s[kt][i] = -INFINITY;
+      }
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, VLO ? fmaf(s[kt][i], c_row, ve[kt][i]) : s[kt][i] * c_row);
+      tmax = max_groups4(tmax);
+      const bool bump = tmax > m_run + 8.0f;
+      if (__any(bump)) {
+        const float m_new = bump ? tmax : m_run;
+        const float corr = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= corr;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] *= corr;
+        m_run = m_new;
+      }
+      const float m_use = (m_run == -INFINITY) ? 0.0f : m_run;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float pv = __builtin_amdgcn_exp2f(fmaf(s[kt][i], c_row, -m_use));
+          pf[kt][i] = pv;
+          const float pp = pv * (VLO ? vp[kt][i] : (float)(1 << kPShift));
+          const _Float16 h = (_Float16)pp;
+          ph[4 * kt + i] = h;
+          pl[4 * kt + i] = (_Float16)(pp - (float)h);
+        }
+      l_run += ((pf[0][0] + pf[0][1]) + (pf[0][2] + pf[0][3])) + ((pf[1][0] + pf[1][1]) + (pf[1][2] + pf[1][3]));
+    }
+
+    // ---- O^T += V^T P^T: 16 dim tiles, two transposing loads per operand
+    {
+      constexpr int D = RD4_PQ_VD;
+      half8 fh[D], fl[D];
+      auto read_v = [&](int dt) RD4_INLINE {
+        const uint8_t *a = vd + v_loff[dt & 7] + 256 * (dt >> 3);
+        auto tr = [](const uint8_t *x) {
+          const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)x);
+          const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(x + 16 * (kHD * 2)));
+          return __builtin_bit_cast(half8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
+        fh[dt % D] = tr(a);
+        if (VLO) fl[dt % D] = tr(a + kPart);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll
+      for (int t = 0; t < D - 1; ++t) read_v(t);
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        if (t + D - 1 < 16) read_v(t + D - 1);
+        if (VFULL) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[t % D], pl, o[t], 0, 0, 0);
+        if (VLO) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[t % D], ph, o[t], 0, 0, 0);
+        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[t % D], pl, o[t], 0, 0, 0);
+        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[t % D], ph, o[t], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // V blocks that are not finite entered as zeros: remembered for the rows that
+    // attend their key
+    if (VLO) {
+      const uint8_t *nf = (const uint8_t *)(tb + 3 * kBN);
+      if (__any(nf[lane & 31] != 0))
+#pragma unroll 1
+        for (int key = 0; key < kBN; ++key)
+          if (j0 + key <= lim_row) poison |= nf[key];
+    }
+    if (isv) next();
+  }
+
+  if (VLO && __any(poison != 0)) {
+#pragma unroll
+    for (int dt = 0; dt < 16; ++dt)
+      if ((poison >> (dt >> 1)) & 1) o[dt] = floatx4{NAN, NAN, NAN, NAN};
+  }
+
+  // ---- epilogue: l over the 4 key groups, then the record of a key split, or
+  // normalize, gate, store
+  float Ls = l_run;
+  Ls += __shfl_xor(Ls, 16, 64);
+  Ls += __shfl_xor(Ls, 32, 64);
+  if (row >= n_rows) return;
+  const int q = row / grp, head = kvh * grp + row % grp;
+  const float o_pw2 = __builtin_ldexpf(1.0f, e0 - kPShift);
+  if (p.n_ksplit > 1) {
+    const int64_t nr = (int64_t)p.n_q * p.n_head, rr = (int64_t)ksp * nr + (int64_t)q * p.n_head + head;
+    float *rec = p.part + rr * kHD;
+#pragma unroll
+    for (int dt = 0; dt < 16; ++dt) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[dt] * o_pw2;
+    if (g == 0) *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run, Ls);
+    return;
+  }
+  const float inv = (m_run == -INFINITY || !(Ls > 0.0f)) ? 0.0f : o_pw2 / Ls;
+  const int64_t ob = ((int64_t)q * p.n_head + head) * kHD;
+#pragma unroll
+  for (int dt = 0; dt < 16; ++dt) {
+    const int d = 16 * dt + 4 * g;
+    float v[4] = {o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv};
+    if (p.gate) {
+      float4 gv = *(const float4 *)(p.gate + ob + d);
+      float gs[4] = {gv.x, gv.y, gv.z, gv.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        gs[i] = 1.0f / (1.0f + expf(-gs[i]));
+        v[i] *= gs[i];
+      }
+      *(float4 *)(p.gate + ob + d) = make_float4(gs[0], gs[1], gs[2], gs[3]);
+    }
+    *(float4 *)(p.out + ob + d) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+}
+
+bool prefill_quant_supported(int kt, int vt, int n_head, int n_head_kv, int head_dim) {
+  const char *e = std::getenv("RD4_PREFILL_GENERIC");
+  if (e && std::atoi(e) != 0) return false;
+  return kt != F32 && vt != F32 && !(kt == F16 && vt == F16) && head_dim == kHD && n_head_kv > 0 &&
+         n_head % n_head_kv == 0;
+}
+
+
+template <bool KLO, bool VLO, bool VFULL = false>
+static void launch(const PrefillArgs &q, dim3 grid, hipStream_t st) {
+  constexpr size_t lds = Lds<KLO, VLO>::kBytes;
+  hipLaunchKernelGGL((prefill_quant_kernel<KLO, VLO, VFULL>), grid, dim3(64 * kW), lds, st, q);
+}
+
+hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st) {
+  PrefillArgs q = p;
+  q.kt = kt;
+  q.vt = vt;
+  const int grp = p.n_head / p.n_head_kv;
+  const int total = (p.n_q * grp + kBM - 1) / kBM * p.n_head_kv;
+  prefill_set_ksplits(q, prefill_ksplits(p, kt, vt, p.part_floats), kBN);
+  dim3 grid((unsigned)(total * q.n_ksplit));
+  if (kt == F16 && vt == Q4_1) launch<false, true, true>(q, grid, st);
+  else if (kt == F16) launch<false, true>(q, grid, st);
+  else if (vt == F16) launch<true, false>(q, grid, st);
+  else if (vt == Q4_1) launch<true, true, true>(q, grid, st);
+  else launch<true, true>(q, grid, st);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || q.n_ksplit == 1) return e;
+  return prefill_merge_launch(q, st);
+}
+
+}  // namespace rd4

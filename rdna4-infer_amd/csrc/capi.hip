@@ -545,8 +545,10 @@ int rd4_attn_split_batch_launch(const float *q, const void *k, const void *v, fl
 // scratch; a call that would split gets it here (without it, no split).
 void prefill_part(PrefillArgs &p, int kt, int vt, hipStream_t st) {
   const uintptr_t al = (uintptr_t)p.q | (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.out | (uintptr_t)p.gate;
-  if ((al & 15) || !prefill_mfma_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim)) return;
-  const int s = prefill_ksplits(p);
+  if ((al & 15) || !(prefill_mfma_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim) ||
+                     prefill_quant_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim)))
+    return;
+  const int s = prefill_ksplits(p, kt, vt, kPartialFloats);
   if (s <= 1 || prefill_part_floats(p, s) > kPartialFloats) return;
   // a stream without a set under graph capture runs unsplit: the lookup's
   // failure is not the call's, so its message is not left behind

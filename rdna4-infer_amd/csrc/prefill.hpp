@@ -31,22 +31,31 @@ struct PrefillArgs {
   int n_ksplit, ksplit_blocks;
   float *part;
   int64_t part_floats;
+  int kt, vt;  // cache types (filled by prefill_quant_launch)
 };
 
 bool prefill_supported(int kt, int vt, int n_head, int n_head_kv, int head_dim);
 hipError_t prefill_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st);
 
+// f16/f16 caches (attn_prefill_mfma.hip) and the quantized pairs
+// (attn_prefill_quant.hip), both head_dim 256.
 bool prefill_mfma_supported(int kt, int vt, int n_head, int n_head_kv, int head_dim);
 hipError_t prefill_mfma_launch(const PrefillArgs &p, hipStream_t st);
-// Key splits the MFMA kernel would run for p (1: none) and the scratch floats
-// their records take; the caller passes the scratch in p.part.
-int prefill_ksplits(const PrefillArgs &p);
+bool prefill_quant_supported(int kt, int vt, int n_head, int n_head_kv, int head_dim);
+hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st);
+// Key splits that the MFMA kernel of this cache pair would run for p (1: none),
+// with records of at most max_floats scratch floats; the caller passes the
+// scratch in p.part.
+int prefill_ksplits(const PrefillArgs &p, int kt, int vt, int64_t max_floats);
 int64_t prefill_part_floats(const PrefillArgs &p, int splits);
+// Fill q's split fields for `splits` splits of key blocks of `bn` keys (1 when
+// q.part cannot hold their records).
+void prefill_set_ksplits(PrefillArgs &q, int splits, int bn);
+// Fold the records of a split call, gate and store.
+hipError_t prefill_merge_launch(const PrefillArgs &q, hipStream_t st);
 
 bool decode_mfma_supported(int kt, int vt, int n_head, int n_head_kv, int head_dim);
 hipError_t decode_mfma_launch(int kt, int vt, const AttnArgs &a, int n_tok, hipStream_t st);
 // True when multi-token decode of this cache pair can put two tokens in a CTA.
 bool decode_mfma_pairs(int kt, int vt);
-// True when split records are merged by a second launch (not the in-kernel tree).
-
 }  // namespace rd4
