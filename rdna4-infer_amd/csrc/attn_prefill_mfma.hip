@@ -34,6 +34,7 @@
 #include <cstdlib>
 
 #include "kv_quant.hpp"
+#include "merge.hpp"
 #include "prefill.hpp"
 
 namespace rd4 {
@@ -232,8 +233,10 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
   // in turn (heaviest first), so an XCD's L2 serves one kv head whose CTAs
   // sweep the same keys at about the same time.
   const int total = n_rb * p.n_head_kv;
-  // key split of this CTA: the splits' grids follow one another, so workgroup
-  // L of a split still runs on XCD L % 8 (total is a multiple of 8 there)
+  // key split of this CTA: the splits' grids follow one another. (With the splits
+  // of a row block as neighbours, an even split count puts each split on its own
+  // XCDs, and causal calls leave some of those idle: 68 -> 77 us at 700 q8_0
+  // queries from position 0.)
   const int ksp = p.n_ksplit > 1 ? (int)blockIdx.x / total : 0;
   const int L = p.n_ksplit > 1 ? (int)blockIdx.x - ksp * total : (int)blockIdx.x;
   int kvh, rbp;
@@ -637,7 +640,7 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
       float *rec = p.part + rr * kHD;
 #pragma unroll
       for (int dt = 0; dt < 16; ++dt)
-        *(floatx4 *)(rec + 16 * dt + 4 * g) = o[sl][dt];
+        if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[sl][dt];  // (m = -inf: the merge drops the record)
       if (g == 0) *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run[sl], L);
       continue;
     }
@@ -664,26 +667,43 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
 
 // Fold of the key splits' records (the LSE merge of the split decode, exp2
 // domain), then the gate and the store of the unsplit epilogue: one wave per
-// (query, head) row, 4 dims per lane.
+// (query, head) row, 4 dims per lane. Bandwidth-bound with many rows and few
+// splits; with few rows and many splits a chain of loads, so lane s loads split
+// s's (m, l), the weights come from lane exchanges, and the records are loaded
+// eight at a time ahead of their use (16 queries, 64 splits: 15 -> 6 us; one
+// load after another before).
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs p) {
   const int lane = threadIdx.x & 63;
   const int64_t nr = (int64_t)p.n_q * p.n_head;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= nr) return;
   const int S = p.n_ksplit;
-  const float *ml = p.part + (int64_t)S * nr * kHD;
-  float M = -INFINITY;
-  for (int s = 0; s < S; ++s) M = fmaxf(M, ml[2 * (s * nr + row)]);
-  float L = 0.0f;
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < S; ++s) {
-    const float2 r = *(const float2 *)(ml + 2 * (s * nr + row));
-    if (r.x == -INFINITY) continue;  // a split with no key of this row
-    const float wgt = __builtin_amdgcn_exp2f(r.x - M);
-    L = fmaf(wgt, r.y, L);
-    const floatx4 v = *(const floatx4 *)(p.part + (s * nr + row) * kHD + 4 * lane);
+  float2 r = make_float2(-INFINITY, 0.0f);
+  if (lane < S) r = *(const float2 *)(p.part + (int64_t)S * nr * kHD + 2 * (lane * nr + row));
+  const float *rec = p.part + row * kHD + 4 * lane;
+  constexpr int kB = 8;
+  floatx4 rv[kB];
+  auto load = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = fmaf(wgt, v[i], acc[i]);
+    for (int i = 0; i < kB; ++i)
+      if (s0 + i < S) rv[i] = *(const floatx4 *)(rec + (int64_t)(s0 + i) * nr * kHD);
+  };
+  load(0);
+  const float M = wave_max(r.x);
+  const float wgt = (r.x == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(r.x - M);
+  const float L = wave_sum(r.x == -INFINITY ? 0.0f : wgt * r.y);
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < S; s0 += kB) {
+    if (s0) load(s0);
+#pragma unroll
+    for (int i = 0; i < kB; ++i) {
+      if (s0 + i >= S) break;
+      // (a split with no key of this row counts for nothing, whatever its record)
+      if (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r.x), s0 + i)) == -INFINITY) continue;
+      const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wgt), s0 + i));
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[c] = fmaf(ws, rv[i][c], acc[c]);
+    }
   }
   const float inv = (M == -INFINITY || !(L > 0.0f)) ? 0.0f : 1.0f / L;
   const int64_t ob = row * kHD + 4 * lane;

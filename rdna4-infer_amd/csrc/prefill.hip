@@ -28,22 +28,35 @@ int compute_units() {
 }
 
 // Rows per CTA and keys per block of a cache pair's MFMA kernel, and what a CTA
-// costs on an MI355X: us per key block, and us before and after its blocks.
+// costs on an MI355X: us per key block (with up to half of the CUs busy, and
+// with all: the f16 kernel's blocks slow down with the clock), and us before and
+// after its blocks.
 struct Shape {
   int rows, keys;
-  double block_us, cta_us;
+  double block_us, block_us_full, cta_us;
 };
 Shape shape_of(int kt, int vt) {
-  if (kt == F16 && vt == F16) return {192, 64, 3.2, 8.0};
-  return {128, 32, 3.4, 8.0};
+  if (kt == F16 && vt == F16) return {192, 64, 2.2, 3.2, 14.0};
+  return {128, 32, 3.3, 3.3, 14.0};
 }
+// The merge launch: us of the launch, and bytes of records written and read per us.
+constexpr double kMergeUs = 3.0, kMergeBytesPerUs = 5e6;
 
 }  // namespace
 
-// A CTA fills a CU, so a call takes ceil(CTAs / CUs) rounds of CTAs. The f16
-// kernel's splits: when its row blocks leave CUs idle (the reference engine's
-// 512-query chunks: 64 CTAs on 256 CUs), about one CTA per CU, at most 16 and
-// at most one per key block. RD4_PREFILL_KSPLIT forces a count (1: never split).
+// Key splits: a CTA fills a CU, so without them a call runs as many CUs as it
+// has row blocks, each over all keys. The count taken is the one of least
+// estimated time: the CTAs of one round all run at once; a further round costs a
+// whole CTA when the rows see about the same keys (a long prefix), and less when
+// they differ (causal rows from position 0, heaviest first); the merge costs its
+// launch and the records' traffic. Measured over split counts 1 to 64 (us: one
+// split / the count taken): f16 201 queries over 1534 keys 76 / 38, 64 over 8064
+// 282 / 42, 16 over 30016 992 / 45, 512 over 8192 288 / 126, 512 over 512 44 /
+// 38, 1000 over 2000 96 / 79; q8_0 16 over 8016 855 / 39, 64 over 1064 126 / 30,
+// 512 over 8192 852 / 391, 512 over 512 74 / 53. The count taken is within 5% of
+// the best in 20 of 24 such calls and within 16% in the others but one (q8_0, 64
+// queries over 8064 keys, whose best count is not a divisor).
+// RD4_PREFILL_KSPLIT forces a count (1: never split).
 int prefill_ksplits(const PrefillArgs &p, int kt, int vt, int64_t max_floats) {
   static const int env = [] {
     const char *e = std::getenv("RD4_PREFILL_KSPLIT");
@@ -53,21 +66,30 @@ int prefill_ksplits(const PrefillArgs &p, int kt, int vt, int64_t max_floats) {
   const int grp = p.n_head / p.n_head_kv;
   const int total = (p.n_q * grp + sh.rows - 1) / sh.rows * p.n_head_kv;
   const int blocks = (p.kmax + sh.keys) / sh.keys;
+  const int most = std::min(blocks, kMaxKSplits);
+  if (env > 0) return std::max(1, std::min(env, most));
   const int cus = compute_units();
-  if (env > 0) return std::max(1, std::min(env, std::min(blocks, 64)));
   if (cus <= 0) return 1;
-  if (kt == F16 && vt == F16)
-    return std::max(1, std::min((total % 8 == 0 && 2 * total <= cus) ? cus / total : 1, std::min(blocks, 16)));
+  // mean blocks of a row: consecutive positions up to kmax
+  const double mean = (std::max(0, p.kmax - p.n_q + 1) + 0.5 * std::min(p.n_q, p.kmax + 1)) / sh.keys;
   int best = 1;
   double best_us = 0;
-  for (int s = 1; s <= std::min(blocks, 64); ++s) {
-    if (s > 1 && prefill_part_floats(p, s) > max_floats) break;
+  for (int s = 1; s <= most; ++s) {
     const int per = (blocks + s - 1) / s;
-    if (s > 1 && (blocks + per - 1) / per != s) continue;
-    const int rounds = (total * s + cus - 1) / cus;
-    double us = rounds * (per * sh.block_us + sh.cta_us);
-    if (s > 1) us += 4.0 + (double)prefill_part_floats(p, s) * 4 / 3.5e6;
-    if (s == 1 || us < best_us) best = s, best_us = us;
+    if (s > 1 && (blocks + per - 1) / per != s) continue;  // as many as a smaller count with the same blocks
+    if (s > 1 && prefill_part_floats(p, s) > max_floats) break;
+    const int64_t ctas = (int64_t)total * s;
+    const double busy = std::min(1.0, std::max(0.0, 2.0 * (double)ctas / cus - 1.0));
+    const double block_us = sh.block_us + (sh.block_us_full - sh.block_us) * busy;
+    const double one = per * block_us + sh.cta_us;
+    const double all = ((double)total * mean * block_us + (double)ctas * sh.cta_us) / cus;
+    const double alike = std::min(1.0, std::max(0.0, 2.0 * mean / blocks - 0.5));
+    const double even = std::max(one, all);
+    double us = even + alike * std::max(0.0, (double)((ctas + cus - 1) / cus) * one - even);
+    if (s > 1) us += kMergeUs + (double)prefill_part_floats(p, s) * 4 / kMergeBytesPerUs;
+    if (s == 1) best_us = 0.9 * us;  // (a split call is two launches: taken for a gain of a tenth or more)
+    else if (us < best_us) best = s, best_us = us;
+    if (ctas > 4 * cus) break;  // more only adds records
   }
   return best;
 }

@@ -47,6 +47,7 @@ hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_
 // with records of at most max_floats scratch floats; the caller passes the
 // scratch in p.part.
 int prefill_ksplits(const PrefillArgs &p, int kt, int vt, int64_t max_floats);
+constexpr int kMaxKSplits = 64;  // the merge gives each split a lane
 int64_t prefill_part_floats(const PrefillArgs &p, int splits);
 // Fill q's split fields for `splits` splits of key blocks of `bn` keys (1 when
 // q.part cannot hold their records).

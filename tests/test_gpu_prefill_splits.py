@@ -1,0 +1,35 @@
+"""Prefill calls whose row blocks leave CUs idle run in key splits that a merge
+launch folds: few queries over many keys (up to the 64 splits a wave of the merge
+holds), row-block counts that are no multiple of 8, splits that hold no key of the
+early rows, and a gate, against the f64 oracle. The f16 path rounds queries and
+probabilities to f16 (the attention tolerance); the quantized path computes in 32
+bits (its tests' tolerance)."""
+import numpy as np
+import pytest
+
+from gpu_util import check_close, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("t", [1, 2])
+@pytest.mark.parametrize("nh,nkv,pos0,nq", [(24, 4, 4100, 1), (24, 4, 4095, 16), (24, 4, 2000, 23), (32, 8, 777, 57),
+                                            (16, 2, 300, 97), (6, 1, 0, 300), (12, 3, 63, 201), (24, 4, 0, 400)])
+def test_split_calls_match_oracle(rd4, orc, dev, t, nh, nkv, pos0, nq):
+    import torch
+    n, seed = pos0 + nq, 13 * pos0 + nq
+    k, v = orc.store_rows(t, orc.randn(n * nkv * 256, seed)), orc.store_rows(t, orc.randn(n * nkv * 256, seed + 1))
+    q, g = orc.randn(nq * nh * 256, seed + 2).reshape(nq, nh, 256), orc.randn(nq * nh * 256, seed + 3).reshape(nq, nh, 256)
+    rows = np.unique(np.linspace(0, nq - 1, 40).astype(np.int32))
+    want = orc.attn_batch(q[rows], k, v, pos0 + rows, nh, nkv, 256, 1 / 16, t, t, threads=8)
+    _, want = orc.sigmoid_gate(g[rows], want)
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=dev)
+    rd4.prefill(to_dev(q, torch, dev), to_dev(k, torch, dev), to_dev(v, torch, dev), out, pos0, nh, nkv, 256, 1 / 16, t, t,
+                gate=to_dev(g, torch, dev))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    assert np.all(np.isfinite(got))
+    check_close(got[rows].ravel(), np.asarray(want).ravel(), "prefill %d/%d pos0 %d n %d" % (nh, nkv, pos0, nq))
+    if t != 1:
+        want = np.asarray(want, np.float64).reshape(got[rows].shape)
+        assert np.linalg.norm(got[rows] - want) <= 3e-6 * np.linalg.norm(want)
