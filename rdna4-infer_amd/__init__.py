@@ -103,12 +103,27 @@ def _check(rc, what):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()  # (the argtypes take an integer as a pointer)
+
+
+_raw_stream = None  # device -> handle of its current stream, and the current device
 
 
 def _stream():
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """Handle of the current stream of the current device. Through
+    torch.cuda.current_stream() the lookup builds a Stream object, 3.0 us of the
+    9.4 us that a one-launch call took on the host; the two bindings under it take
+    0.2 us."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        torch.cuda.current_stream()  # initialises the runtime
+        get, dev = getattr(torch._C, "_cuda_getCurrentRawStream", None), getattr(torch._C, "_cuda_getDevice", None)
+        if get is None or dev is None:
+            _raw_stream = (lambda d: torch.cuda.current_stream().cuda_stream), (lambda: 0)
+        else:
+            _raw_stream = get, dev
+    return _raw_stream[0](_raw_stream[1]())
 
 
 # ---- KV tables (kv.h:100-169) ------------------------------------------------
