@@ -34,12 +34,16 @@
 // Two stages, one CTA barrier per block. Waves w and w + 4 share a SIMD:
 // waves 0-3 convert before their products, 4-7 after, so that one's conversion
 // runs beside the other's matrix instructions.
-// What bounds it: LDS reads (64 KiB per wave and block, 0.5 MiB per CTA) and the
-// matrix pipe, which takes three products where f16 takes one. 512 queries over
-// 8192 q8_0 keys, 24 / 4 heads: 6120 us in the VALU kernel, 389 us here (0.26
-// PFLOP/s, 0.78 of them counted as issued).
+// What bounds it: LDS reads (64 KiB per wave and block, 0.5 MiB per CTA, 1.1 us
+// of a block's 3.0) and the matrix pipe (192 products per SIMD and block, 1.5 us),
+// which two waves per SIMD overlap in part; the conversion is 0.6 us of it. 512
+// queries over 8192 q8_0 keys, 24 / 4 heads: 6120 us in the VALU kernel, 350 us
+// here (0.28 PFLOP/s, 0.85 counted as issued). Conversion pieces between the
+// products of a block, one pair after each fragment, were slower than in one go
+// at opposite ends of the block for the two waves of a SIMD (350 against 340 us).
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "kv_quant.hpp"
 #include "prefill.hpp"
@@ -101,13 +105,20 @@ __device__ __forceinline__ float max_groups4(float x) {
   __asm__("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
   return fmaxf(c, d);
 }
-// unsigned max over the 8 lanes 8k .. 8k + 7
-__device__ __forceinline__ uint32_t max8_u32(uint32_t x) {
+// Row and block of a lane in the conversion of a wave's 8 rows: 16 consecutive
+// lanes hold blocks 4h .. 4h + 3 of rows 0, 2, 4, 6 (or 1, 3, 5, 7), whose chunks
+// i of the 16-byte swizzle fall in 16 different slots: the stage writes meet no
+// bank conflict (8 lanes per row in order: 2-way).
+__device__ __forceinline__ int conv_row(int lane) { return ((lane >> 4) & 1) | (((lane >> 2) & 3) << 1); }
+__device__ __forceinline__ int conv_block(int lane) { return (lane & 3) | ((lane >> 5) << 2); }
+// unsigned max over the 8 lanes of a row
+__device__ __forceinline__ uint32_t max_row_u32(uint32_t x) {
   int v = (int)x;
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
-  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));  // row_half_mirror
-  return (uint32_t)v;
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));  // quad_perm 1,0,3,2
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));  // quad_perm 2,3,0,1
+  int c = v, d = v;
+  __asm__("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
+  return (uint32_t)max(c, d);
 }
 
 // 16 bytes per lane from sbase + voff into LDS at lds + 16 * lane (asm, so the
@@ -171,55 +182,48 @@ __device__ __forceinline__ void block_words(const uint8_t *row, int b, uint32_t 
   }
 }
 
+// Elements 2f, 2f + 1 of the block whose words block_words read: an f16 pair of
+// the integers (exact), T's bias taken off.
 template <int T>
-__device__ __forceinline__ void convert_words(const uint32_t *w, half2v d, half2v m, uint32_t hi[16], uint32_t lo[16]) {
-  if constexpr (T == Q8_0) {
-    // f16 1024 + 128 + byte, less 1152 (exact)
+__device__ __forceinline__ half2v block_pair(const uint32_t *w, int f) {
+  if constexpr (T == Q8_0) {  // f16 1024 + 128 + byte, less 1152
     const half2v c = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      split_mul(as_h2(__builtin_amdgcn_perm(0u, w[i], 0x0c010c00u) ^ 0x64806480u) + c, d, hi[2 * i], lo[2 * i]);
-      split_mul(as_h2(__builtin_amdgcn_perm(0u, w[i], 0x0c030c02u) ^ 0x64806480u) + c, d, hi[2 * i + 1], lo[2 * i + 1]);
-    }
+    return as_h2(__builtin_amdgcn_perm(0u, w[f >> 1], (f & 1) ? 0x0c030c02u : 0x0c010c00u) ^ 0x64806480u) + c;
   } else {
-    constexpr int W0 = T == Q5_0 ? 1 : 0;
     constexpr float kBias = T == Q4_0 ? -1032.0f : T == Q5_0 ? -1040.0f : -1024.0f;
     const half2v c = {(_Float16)kBias, (_Float16)kBias};
-#pragma unroll
-    for (int half = 0; half < 2; ++half)  // low nibbles: elements 0..15, high: 16..31
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {       // elements 16 half + 2i, 2i + 1: bytes 2i, 2i + 1
-        const uint32_t by = __builtin_amdgcn_perm(0u, w[W0 + (i >> 1)], (i & 1) ? 0x0c030c02u : 0x0c010c00u);
-        uint32_t n = (half ? by >> 4 : by) & 0x000f000fu;
-        if constexpr (T == Q5_0) {
-          const uint32_t hb = w[0] >> (16 * half + 2 * i);  // bits of the two elements
-          n |= ((hb & 1u) << 4) | ((hb & 2u) << 19);
-        }
-        const half2v q = as_h2(n | 0x64006400u) + c;
-        if constexpr (T == Q4_1) split_mul_add(q, d, m, hi[8 * half + i], lo[8 * half + i]);
-        else split_mul(q, d, hi[8 * half + i], lo[8 * half + i]);
-      }
+    const int half = f >> 3, i = f & 7;  // low nibbles: elements 0..15, high: 16..31
+    const uint32_t by = __builtin_amdgcn_perm(0u, w[(T == Q5_0 ? 1 : 0) + (i >> 1)], (i & 1) ? 0x0c030c02u : 0x0c010c00u);
+    uint32_t n = (half ? by >> 4 : by) & 0x000f000fu;
+    if constexpr (T == Q5_0) {
+      const uint32_t hb = w[0] >> (16 * half + 2 * i);  // bits of the two elements
+      n |= ((hb & 1u) << 4) | ((hb & 2u) << 19);
+    }
+    return as_h2(n | 0x64006400u) + c;
   }
 }
 
 // Exponent of a row's power of two, from the f16 magnitude bits of its blocks'
 // scales (one per lane of the row's 8; the largest finite one counts).
 __device__ __forceinline__ int row_exponent(uint32_t mag) {
-  return max((int)(max8_u32(mag >= 0x7c00u ? 0u : mag) >> 10), 1) - 15;
+  return max((int)(max_row_u32(mag >= 0x7c00u ? 0u : mag) >> 10), 1) - 15;
 }
 
-// Convert the wave's 8 raw rows (lane = 8 * row + block) to the hi / lo stage.
-template <int T>
-__device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int lane, uint8_t *hi_st, uint8_t *lo_st,
-                                             float *pw2_tab, float *exp_tab, uint8_t *nf_tab, int e0) {
-  const int r = lane >> 3, b = lane & 7, key = key0 + r;
-  const int dst = key * (kHD * 2), sz = swz(key & 15);
+// Convert the wave's 8 raw rows (lane: row conv_row, block conv_block; rb bytes per
+// row) into the stage rows at hi_st (their lo parts kPart bytes on) and the tables:
+// pw2_tab[key] = 2^(e - e0 + shift), and for V exp_tab[key] = e - e0 and
+// nf_tab[key] = the mask of blocks that are not finite.
+template <int T, bool V>
+__device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int lane, uint8_t *hi_st, float *pw2_tab,
+                                             float *exp_tab, uint8_t *nf_tab, int e0) {
+  const int r = conv_row(lane), b = conv_block(lane), key = key0 + r, sz = swz(key & 15);
+  uint8_t *dst = hi_st + key * (kHD * 2);
   if constexpr (T == F16) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      *(u32x4 *)(hi_st + dst + 16 * ((4 * b + i) ^ sz)) = *(const u32x4 *)(raw + r * 512 + 64 * b + 16 * i);
+      *(u32x4 *)(dst + 16 * ((4 * b + i) ^ sz)) = *(const u32x4 *)(raw + r * 512 + 64 * b + 16 * i);
   } else {
-    uint32_t w[8], dm, hi[16], lo[16];
+    uint32_t w[8], dm, ch[4], cl[4];
     block_words<T>(raw + r * (8 * block_bytes(T)), b, w, &dm);
     // The row's power of two from its largest scale (q4_1: or offset) magnitude.
     uint32_t mag = dm & 0x7fffu;
@@ -231,23 +235,25 @@ __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int l
     // A block that is not finite: K keeps it (its keys' scores become NaN). V's
     // enters the products as zeros, so that rows which do not attend the key keep
     // their sums; nf_tab marks it, and the rows that attend the key end as NaN.
-    if (exp_tab && nonfin) d = (_Float16)0.0f, m = (_Float16)0.0f;
-    convert_words<T>(w, half2v{d, d}, half2v{m, m}, hi, lo);
+    if (V && nonfin) d = (_Float16)0.0f, m = (_Float16)0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int off = dst + 16 * ((4 * b + i) ^ sz);
-      *(u32x4 *)(hi_st + off) = u32x4{hi[4 * i], hi[4 * i + 1], hi[4 * i + 2], hi[4 * i + 3]};
-      *(u32x4 *)(lo_st + off) = u32x4{lo[4 * i], lo[4 * i + 1], lo[4 * i + 2], lo[4 * i + 3]};
-    }
-    if (exp_tab) {
-      const uint64_t nf = __ballot(nonfin);
-      if (b == 0) {
-        pw2_tab[key] = __builtin_ldexpf(1.0f, e - e0 + kPShift);
-        exp_tab[key] = (float)(e - e0);
-        nf_tab[key] = (uint8_t)(nf >> (8 * r));
+    for (int f = 0; f < 16; ++f) {
+      const half2v q = block_pair<T>(w, f);
+      if constexpr (T == Q4_1) split_mul_add(q, half2v{d, d}, half2v{m, m}, ch[f & 3], cl[f & 3]);
+      else split_mul(q, half2v{d, d}, ch[f & 3], cl[f & 3]);
+      if ((f & 3) == 3) {
+        uint8_t *at = dst + 16 * ((4 * b + (f >> 2)) ^ sz);
+        *(u32x4 *)at = u32x4{ch[0], ch[1], ch[2], ch[3]};
+        *(u32x4 *)(at + kPart) = u32x4{cl[0], cl[1], cl[2], cl[3]};
       }
-    } else if (b == 0) {
-      pw2_tab[key] = __builtin_ldexpf(1.0f, e);
+    }
+    const uint64_t nf = __ballot(nonfin);
+    if (b == 0) {
+      pw2_tab[key] = __builtin_ldexpf(1.0f, V ? e - e0 + kPShift : e);
+      if (V) {
+        exp_tab[key] = (float)(e - e0);
+        nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
+      }
     }
   }
 }
@@ -258,17 +264,15 @@ __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int l
 #define RD4_INLINE __attribute__((always_inline))
 
 // K fragments and V operand pairs in registers or in flight ahead of their products
-#ifndef RD4_PQ_KD
-#define RD4_PQ_KD 3
-#endif
-#ifndef RD4_PQ_VD
-#define RD4_PQ_VD 3
-#endif
+constexpr int kRing = 3;  // (2 to 5: within 1%)
 
-// KLO, VLO: the rows have remainder parts (all but f16); VFULL: q4_1 values, whose
-// remainders are as full as p's, take the fourth product vl.pl too (at 120 queries
-// over 120 keys the error is 1.04 times the VALU kernel's without it, 0.88 with).
-template <bool KLO, bool VLO, bool VFULL>
+// KT, VT: the cache types, or -1 for a type read at run time. KLO, VLO: the rows
+// have remainder parts (all but f16); VFULL: q4_1 values, whose remainders are as
+// full as p's, take the fourth product vl.pl too (at 120 queries over 120 keys the
+// error is 1.04 times the VALU kernel's without it, 0.88 with).
+template <int T>
+using type_c = std::integral_constant<int, T>;
+template <int KT, int VT, bool KLO, bool VLO, bool VFULL>
 __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p) {
   using L = Lds<KLO, VLO>;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -316,53 +320,58 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   const uint8_t *my_base = (isv ? p.v : p.k) + (int64_t)kvh * rb;
   const int my_stride = p.n_head_kv * rb;
   uint8_t *raw = smem + L::kRaw + (isv ? 4 * L::kRawK + (w - 4) * L::kRawV : w * L::kRawK);
-  int c_key[4], c_off[4];  // key in the block and byte in its row of each 16-byte chunk
+  uint32_t c_at[4];  // key in the block (high half) and byte in its row of each 16-byte chunk
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = min(64 * i + lane, 8 * nch - 1);  // (surplus lanes repeat the last chunk into the padding)
-    c_key[i] = 8 * (w & 3) + c / nch;
-    c_off[i] = 16 * (c % nch);
+    c_at[i] = (uint32_t)(8 * (w & 3) + c / nch) << 16 | (uint32_t)(16 * (c % nch));
   }
   auto issue = [&](int bi) RD4_INLINE {
     const int j0 = (b0 + bi) * kBN;
     const uint8_t *src = uniform_ptr(my_base + (int64_t)j0 * my_stride);
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // keys past kend re-read a valid row (masked later)
-      if (i < n_dma) dma16(src, (uint32_t)(min(c_key[i], kend - j0) * my_stride + c_off[i]), lds_addr(raw + 1024 * i));
+      if (i < n_dma) dma16(src, (uint32_t)(min((int)(c_at[i] >> 16), kend - j0) * my_stride) + (c_at[i] & 0xffffu), lds_addr(raw + 1024 * i));
   };
   // O and p * 2^e are kept relative to the exponent of the CTA's first V row, so
   // that p itself is near 1 where it matters (the argument of its exp2 near 0)
   int e0 = 0;
   if (VLO && nbk > 0) {
     const int vrb = (int)row_bytes(p.vt, kHD);
-    const uint8_t *blk = p.v + ((int64_t)b0 * kBN * p.n_head_kv + kvh) * vrb + (lane & 7) * (vrb >> 3);
+    const uint8_t *blk = p.v + ((int64_t)b0 * kBN * p.n_head_kv + kvh) * vrb + conv_block(lane) * (vrb >> 3);
     uint32_t mag = ld_u16(blk) & 0x7fffu;
     if (p.vt == Q4_1) mag = max(mag, (uint32_t)ld_u16(blk + 2) & 0x7fffu);
     e0 = __builtin_amdgcn_readfirstlane(row_exponent(mag));
   }
   auto tab = [&](int st) RD4_INLINE { return (float *)(smem + L::kTab + st * L::kTabStage); };
-  auto convert = [&](int st) RD4_INLINE {
-    uint8_t *sb = smem + st * L::kStage;
+  auto convert_as = [&](auto type, auto is_v, int st) RD4_INLINE {
     float *t = tab(st);
-    const int key0 = 8 * (w & 3);
-    if (!isv) {
-      if constexpr (!KLO) convert_rows<F16>(raw, key0, lane, sb + L::KH, nullptr, t, nullptr, nullptr, 0);
-      else switch (p.kt) {
-        case Q8_0: convert_rows<Q8_0>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
-        case Q4_0: convert_rows<Q4_0>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
-        case Q5_0: convert_rows<Q5_0>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
-        default: convert_rows<Q4_1>(raw, key0, lane, sb + L::KH, sb + L::KL, t, nullptr, nullptr, 0); break;
-      }
-    } else {
-      float *vp = t + kBN, *ve = t + 2 * kBN;
-      uint8_t *nf = (uint8_t *)(t + 3 * kBN);
-      if constexpr (!VLO) convert_rows<F16>(raw, key0, lane, sb + L::VH, nullptr, vp, ve, nf, e0);
-      else switch (p.vt) {
-        case Q8_0: convert_rows<Q8_0>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
-        case Q4_0: convert_rows<Q4_0>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
-        case Q5_0: convert_rows<Q5_0>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
-        default: convert_rows<Q4_1>(raw, key0, lane, sb + L::VH, sb + L::VL, vp, ve, nf, e0); break;
-      }
+    uint8_t *sb = smem + st * L::kStage;
+    constexpr int T = decltype(type)::value;
+    if constexpr (decltype(is_v)::value)
+      convert_rows<T, true>(raw, 8 * (w & 3), lane, sb + L::VH, t + kBN, t + 2 * kBN, (uint8_t *)(t + 3 * kBN), e0);
+    else
+      convert_rows<T, false>(raw, 8 * (w & 3), lane, sb + L::KH, t, nullptr, nullptr, 0);
+  };
+  // this wave's rows into stage st: K for waves 0-3, V for 4-7
+  auto convert_k = [&](int st) RD4_INLINE {
+    if constexpr (KT >= 0) convert_as(type_c<KT>{}, std::false_type{}, st);
+    else if constexpr (!KLO) convert_as(type_c<F16>{}, std::false_type{}, st);
+    else switch (p.kt) {
+      case Q8_0: convert_as(type_c<Q8_0>{}, std::false_type{}, st); break;
+      case Q4_0: convert_as(type_c<Q4_0>{}, std::false_type{}, st); break;
+      case Q5_0: convert_as(type_c<Q5_0>{}, std::false_type{}, st); break;
+      default: convert_as(type_c<Q4_1>{}, std::false_type{}, st); break;
+    }
+  };
+  auto convert_v = [&](int st) RD4_INLINE {
+    if constexpr (VT >= 0) convert_as(type_c<VT>{}, std::true_type{}, st);
+    else if constexpr (!VLO) convert_as(type_c<F16>{}, std::true_type{}, st);
+    else if constexpr (VFULL) convert_as(type_c<Q4_1>{}, std::true_type{}, st);
+    else switch (p.vt) {
+      case Q8_0: convert_as(type_c<Q8_0>{}, std::true_type{}, st); break;
+      case Q4_0: convert_as(type_c<Q4_0>{}, std::true_type{}, st); break;
+      default: convert_as(type_c<Q5_0>{}, std::true_type{}, st); break;
     }
   };
   if (nbk > 0) issue(0);
@@ -432,17 +441,19 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   const int tr_kx = 4 * g + (n >> 2);
   const int tr_off = tr_kx * (kHD * 2) + 8 * (n & 1);
   const int tr_m = 16 * ((n >> 1 & 1) ^ swz(tr_kx));
-  int v_loff[8], k_loff[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    v_loff[i] = tr_off + ((32 * i) ^ tr_m);
-    k_loff[i] = n * (kHD * 2) + 16 * ((4 * i + g) ^ swz(n));
-  }
+  // LDS address of fragment 0 in stage 0; the others differ in XORed bits (the
+  // stages are 512-byte aligned), which costs an instruction at each read and no
+  // registers
+  auto lds_of = [](const uint8_t *x) RD4_INLINE { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)x; };
+  const uint32_t v_at = lds_of(smem + L::VH) + tr_off + tr_m;
+  const uint32_t k_at = lds_of(smem + L::KH) + n * (kHD * 2) + 16 * (g ^ swz(n));
 
   // the first block's rows: converted before the loop
   if (nbk > 0) {
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    convert(0);
+    if (isv) convert_v(0);
+    else convert_k(0);
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // raw rows read before they are overwritten
     if (nbk > 1) issue(1);
   }
 
@@ -453,31 +464,30 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     // block bi is written; past the barrier so is every wave's, and all are done
     // reading the other stage
     __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    auto next = [&]() RD4_INLINE {
-      if (bi + 1 < nbk) {
-        convert(st ^ 1);
-        __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // raw rows read before they are overwritten
-        if (bi + 2 < nbk) issue(bi + 2);
-      }
+    const bool more = bi + 1 < nbk;
+    auto refill = [&]() RD4_INLINE {
+      __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // raw rows read before they are overwritten
+      if (bi + 2 < nbk) issue(bi + 2);
     };
-    if (!isv) next();
-    const uint8_t *kd = smem + st * L::kStage + L::KH;
-    const uint8_t *vd = smem + st * L::kStage + L::VH;
+    if (more && !isv) {
+      convert_k(st ^ 1);
+      refill();
+    }
+    const uint32_t k_st = k_at + st * L::kStage, v_st = v_at + st * L::kStage;
     const float *tb = tab(st);
 
-    // ---- S^T of the two 16-key tiles: fragment f = (dim block f / 2, tile f % 2)
-    // (the small products in a sum of their own and the large ones in four, so that
-    // few roundings happen at the size of the whole sum)
-    floatx4 sc[2][5], s[2];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) sc[i / 5][i % 5] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // ---- S^T of the two 16-key tiles: fragment f = (tile f / 8, dim block f % 8).
+    // (The small products go to a sum of their own and the large ones to four, so
+    // that few roundings happen at the size of the whole sum.)
+    floatx4 s[2];
     {
-      constexpr int D = RD4_PQ_KD;
+      constexpr int D = kRing;
       u32x4 fh[D], fl[D];
+      floatx4 sc[5];
       auto read_k = [&](int f) RD4_INLINE {
-        const uint8_t *a = kd + (f & 1) * 16 * (kHD * 2) + k_loff[f >> 1];
-        fh[f % D] = *(const lds_u32x4 *)a;
-        if (KLO) fl[f % D] = *(const lds_u32x4 *)(a + kPart);
+        const uint32_t a = (k_st ^ (64u * (f & 7))) + (f >> 3) * 16 * (kHD * 2);
+        fh[f % D] = *(lds_u32x4 *)a;
+        if (KLO) fl[f % D] = *(lds_u32x4 *)(a + kPart);
         __builtin_amdgcn_sched_barrier(0);
       };
 #pragma unroll
@@ -485,19 +495,20 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
 #pragma unroll
       for (int f = 0; f < 16; ++f) {
         if (f + D - 1 < 16) read_k(f + D - 1);
-        const int b = f >> 1, kt = f & 1;
+        const int b = f & 7, kt = f >> 3;
+        if (b == 0) {
+#pragma unroll
+          for (int i = 0; i < 5; ++i) sc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
         const half8 kh = __builtin_bit_cast(half8, fh[f % D]);
-        floatx4 &sl = sc[kt][4];
-        if (KLO) sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, fl[f % D]), qh[b], sl, 0, 0, 0);
-        sl = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[b], sl, 0, 0, 0);
-        sc[kt][b & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[b], sc[kt][b & 3], 0, 0, 0);
+        if (KLO) sc[4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, fl[f % D]), qh[b], sc[4], 0, 0, 0);
+        sc[b & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[b], sc[b & 3], 0, 0, 0);
+        sc[4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[b], sc[4], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b == 7) s[kt] = ((sc[0] + sc[1]) + (sc[2] + sc[3])) + sc[4];
       }
     }
-
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt) s[kt] = ((sc[kt][0] + sc[kt][1]) + (sc[kt][2] + sc[kt][3])) + sc[kt][4];
-
     // ---- online softmax: lane = row n, keys 16 kt + 4 g + i. The running max
     // (m_run, in log2) follows s + e (e: the V row's exponent), which bounds p * 2^e.
     half8 ph, pl;
@@ -555,11 +566,11 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
 
     // ---- O^T += V^T P^T: 16 dim tiles, two transposing loads per operand
     {
-      constexpr int D = RD4_PQ_VD;
+      constexpr int D = kRing;
       half8 fh[D], fl[D];
       auto read_v = [&](int dt) RD4_INLINE {
-        const uint8_t *a = vd + v_loff[dt & 7] + 256 * (dt >> 3);
-        auto tr = [](const uint8_t *x) {
+        const uint32_t a = v_st ^ (32u * dt);
+        auto tr = [](uint32_t x) RD4_INLINE {
           const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)x);
           const short4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(x + 16 * (kHD * 2)));
           return __builtin_bit_cast(half8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -580,6 +591,10 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+    if (more && isv) {
+      convert_v(st ^ 1);
+      refill();
+    }
     // V blocks that are not finite entered as zeros: remembered for the rows that
     // attend their key
     if (VLO) {
@@ -589,7 +604,6 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
         for (int key = 0; key < kBN; ++key)
           if (j0 + key <= lim_row) poison |= nf[key];
     }
-    if (isv) next();
   }
 
   if (VLO && __any(poison != 0)) {
@@ -643,10 +657,10 @@ bool prefill_quant_supported(int kt, int vt, int n_head, int n_head_kv, int head
 }
 
 
-template <bool KLO, bool VLO, bool VFULL = false>
+template <int KT, int VT, bool KLO = KT != F16, bool VLO = VT != F16, bool VFULL = VT == Q4_1>
 static void launch(const PrefillArgs &q, dim3 grid, hipStream_t st) {
   constexpr size_t lds = Lds<KLO, VLO>::kBytes;
-  hipLaunchKernelGGL((prefill_quant_kernel<KLO, VLO, VFULL>), grid, dim3(64 * kW), lds, st, q);
+  hipLaunchKernelGGL((prefill_quant_kernel<KT, VT, KLO, VLO, VFULL>), grid, dim3(64 * kW), lds, st, q);
 }
 
 hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st) {
@@ -657,11 +671,19 @@ hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_
   const int total = (p.n_q * grp + kBM - 1) / kBM * p.n_head_kv;
   prefill_set_ksplits(q, prefill_ksplits(p, kt, vt, p.part_floats), kBN);
   dim3 grid((unsigned)(total * q.n_ksplit));
-  if (kt == F16 && vt == Q4_1) launch<false, true, true>(q, grid, st);
-  else if (kt == F16) launch<false, true>(q, grid, st);
-  else if (vt == F16) launch<true, false>(q, grid, st);
-  else if (vt == Q4_1) launch<true, true, true>(q, grid, st);
-  else launch<true, true>(q, grid, st);
+  // the pairs that caches are made of have their conversion built in; the others
+  // switch on the type in each block (q8_0, 512 queries over 8192 keys: 350 us
+  // built in, 384 switched)
+  if (kt == Q8_0 && vt == Q8_0) launch<Q8_0, Q8_0>(q, grid, st);
+  else if (kt == Q4_0 && vt == Q4_0) launch<Q4_0, Q4_0>(q, grid, st);
+  else if (kt == Q5_0 && vt == Q5_0) launch<Q5_0, Q5_0>(q, grid, st);
+  else if (kt == Q4_1 && vt == Q4_1) launch<Q4_1, Q4_1>(q, grid, st);
+  else if (kt == Q5_0 && vt == Q4_1) launch<Q5_0, Q4_1>(q, grid, st);
+  else if (kt == F16 && vt == Q4_1) launch<F16, -1, false, true, true>(q, grid, st);
+  else if (kt == F16) launch<F16, -1, false, true, false>(q, grid, st);
+  else if (vt == F16) launch<-1, F16, true, false, false>(q, grid, st);
+  else if (vt == Q4_1) launch<-1, -1, true, true, true>(q, grid, st);
+  else launch<-1, -1, true, true, false>(q, grid, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || q.n_ksplit == 1) return e;
   return prefill_merge_launch(q, st);

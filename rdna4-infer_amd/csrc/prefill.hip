@@ -37,7 +37,7 @@ struct Shape {
 };
 Shape shape_of(int kt, int vt) {
   if (kt == F16 && vt == F16) return {192, 64, 2.2, 3.2, 14.0};
-  return {128, 32, 3.3, 3.3, 14.0};
+  return {128, 32, 3.0, 3.0, 14.0};
 }
 // The merge launch: us of the launch, and bytes of records written and read per us.
 constexpr double kMergeUs = 3.0, kMergeBytesPerUs = 5e6;
@@ -53,7 +53,7 @@ constexpr double kMergeUs = 3.0, kMergeBytesPerUs = 5e6;
 // split / the count taken): f16 201 queries over 1534 keys 76 / 38, 64 over 8064
 // 282 / 42, 16 over 30016 992 / 45, 512 over 8192 288 / 126, 512 over 512 44 /
 // 38, 1000 over 2000 96 / 79; q8_0 16 over 8016 855 / 39, 64 over 1064 126 / 30,
-// 512 over 8192 852 / 391, 512 over 512 74 / 53. The count taken is within 5% of
+// 512 over 8192 852 / 350, 512 over 512 74 / 50. The count taken is within 5% of
 // the best in 20 of 24 such calls and within 16% in the others but one (q8_0, 64
 // queries over 8064 keys, whose best count is not a divisor).
 // RD4_PREFILL_KSPLIT forces a count (1: never split).
@@ -117,7 +117,7 @@ hipError_t prefill_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st) 
   // A call with few keys is all launch and first-use latency, and the VALU
   // kernel's is shorter: 16 queries over 16 q8_0 keys 17.2 us there, 18.9 us on
   // the matrix cores; 64 over 64 30.8 against 24.1 us, 512 over 8192 6121
-  // against 384 us.
+  // against 350 us.
   if ((al & 15) == 0 && p.kmax >= 24 && prefill_quant_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim))
     return prefill_quant_launch(kt, vt, p, st);
   AttnArgs a{};
