@@ -79,6 +79,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kHD = 256;     // head_dim of this kernel
 constexpr int kRowPad = kHD + 4;  // LDS row stride (floats) of per-head rows: spreads banks
 constexpr int kTile = 16;    // keys per wave tile
+constexpr int kEvenTiles = 16;  // tiles of a CTA dealt to all 8 waves alike
 constexpr int kG = 8;        // query heads per CTA (MFMA rows 0-7 hi, 8-15 lo)
 constexpr float kLog2e = 1.4426950408889634f;
 // int8 query image (q8_0 K): rows [16][8 blocks][32] padded to kQiRow bytes,
@@ -859,6 +860,51 @@ __global__ __launch_bounds__((64 * TileShape<KT, VT>::WAVES), 1) void decode_mfm
   const uint8_t *kbase = a.k + (int64_t)kvh * rowb<KT>();
   const uint8_t *vbase = a.v + (int64_t)kvh * rowb<VT>();
 
+  // The chunk's G query rows are copied into LDS once per CTA by the same
+  // global->LDS DMA, issued before any tile so they are not queued behind the
+  // tiles; rows are padded by 16 bytes so the per-row fragment reads below do
+  // not collide in one bank.
+  uint8_t *q_lds = smem + kWaves * (R * TB);
+  const int qcw = a.q_f16 ? kHD / 8 : kHD / 4;  // 16-byte chunks per query row
+  const int qsb = 16 * (qcw + 1);               // padded row stride in bytes
+  auto issue_q = [&]() {  // one load instruction per 64 chunks, spread over the waves
+    if (RD4_DEC_KNOBS && (a.dbg & 2048)) return;
+    for (int base = 64 * w; base < G * (qcw + 1); base += 64 * kWaves) {
+      const int idx = base + lane, r = idx / (qcw + 1), c = idx - r * (qcw + 1);
+      if (r < G && c < qcw) {
+        const uint8_t *src = (const uint8_t *)a.q +
+                             (((int64_t)tok * a.n_head + h0 + r) * kHD) * (a.q_f16 ? 2 : 4) + 16 * c;
+        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(q_lds + 16 * base), 16, 0, 0);
+      }
+    }
+  };
+  // int8 query path: wave w loads the rows it quantizes straight into registers
+  // (lane l: dims 4l..4l+3), ahead of its tile loads, so it waits for its own
+  // rows only, with no barrier and no LDS traffic
+  float xq[kI8 ? 8 / kWaves : 1][4];
+  auto load_q_own = [&]() {
+#pragma unroll
+    for (int m = 0; m < 8 / kWaves; ++m) {
+      const int r = w + kWaves * m;
+      const int64_t off = ((int64_t)tok * a.n_head + h0 + (r < G ? r : 0)) * kHD + 4 * lane;
+      if (a.q_f16) {
+        const uint2 hv = *(const uint2 *)((const uint16_t *)a.q + off);
+        xq[m][0] = h2f((uint16_t)hv.x);
+        xq[m][1] = h2f((uint16_t)(hv.x >> 16));
+        xq[m][2] = h2f((uint16_t)hv.y);
+        xq[m][3] = h2f((uint16_t)(hv.y >> 16));
+      } else {
+        const float4 fv = *(const float4 *)(a.q + off);
+        xq[m][0] = fv.x;
+        xq[m][1] = fv.y;
+        xq[m][2] = fv.z;
+        xq[m][3] = fv.w;
+      }
+    }
+  };
+  // (int8 query path: these loads run beside the append's in the CTA that owns the
+  // new row. The staged queries go out after the append, which measured 1% faster.)
+  if constexpr (kI8) load_q_own();
   // Fused append: the CTA owning key t writes the new K/V row of its kv head
   // (8-lane groups per 32-element block, the store kernel's quantizer) before
   // any of its tiles is requested; every other CTA starts its loads at once.
@@ -902,14 +948,20 @@ __global__ __launch_bounds__((64 * TileShape<KT, VT>::WAVES), 1) void decode_mfm
   const int n_tiles_all = j_end > j_begin ? (j_end - j_begin - 1) / j_step + 1 : 0;
   // Tile order: with 8 waves, waves w and w + 4 share a SIMD and the older one
   // (w < 4) is issued first, so it takes more tiles: n_lo rounds go to all 8
-  // waves (tile 8i + w), the rest to waves 0-3 only (4 per round).
+  // waves (tile 8i + w), the rest to waves 0-3 only (4 per round). Up to
+  // kEvenTiles the tiles go round all 8 waves instead: a CTA with 5 tiles waits
+  // for one in each wave and not for two in waves 0-3 (per layer, with the int8
+  // queries loaded ahead of the append: 5001 keys q8_0 13.6 -> 12.3 us, q4_0 13.3
+  // -> 12.6, q5_0 / q4_1 15.3 -> 14.3; 9000 keys 15.5 -> 14.3, 15.1 -> 14.1, 17.7
+  // -> 16.0; 777 and 32768 keys the same).
 #ifndef RD4_DEC_LO
 #define RD4_DEC_LO 6
 #endif
-  const int n_lo = kWaves == 8 ? n_tiles_all * RD4_DEC_LO / 64 : n_tiles_all;
-  const int t_rem = kWaves == 8 ? n_tiles_all - 8 * n_lo : 0;
+  const int n_lo = kWaves != 8 ? n_tiles_all
+                   : n_tiles_all <= kEvenTiles ? (n_tiles_all + 7) / 8 : n_tiles_all * RD4_DEC_LO / 64;
+  const int t_rem = kWaves == 8 ? n_tiles_all - 8 * n_lo : 0;  // (below 0 in an uneven last round)
   const int my_tiles = (RD4_DEC_KNOBS && (a.dbg & 32)) ? 0
-                       : kWaves == 8 ? (w < 4 ? n_lo + (t_rem > w ? (t_rem - w + 3) / 4 : 0) : n_lo)
+                       : kWaves == 8 ? min(n_lo, (n_tiles_all - w + 7) >> 3) + (w < 4 && t_rem > w ? (t_rem - w + 3) / 4 : 0)
                                      : (n_tiles_all > w ? (n_tiles_all - w + kWaves - 1) / kWaves : 0);
   auto tile_of = [&](int i) {
     return kWaves == 8 ? (i < n_lo ? 8 * i + w : 8 * n_lo + 4 * (i - n_lo) + w) : w + i * kWaves;
@@ -969,52 +1021,7 @@ __global__ __launch_bounds__((64 * TileShape<KT, VT>::WAVES), 1) void decode_mfm
                                            (lds_void *)(st + 1024 * r), 16, 0, kAux);
     }
   };
-  // The chunk's G query rows are copied into LDS once per CTA by the same
-  // global->LDS DMA, issued before any tile so they are not queued behind the
-  // tiles; rows are padded by 16 bytes so the per-row fragment reads below do
-  // not collide in one bank.
-  uint8_t *q_lds = smem + kWaves * (R * TB);
-  const int qcw = a.q_f16 ? kHD / 8 : kHD / 4;  // 16-byte chunks per query row
-  const int qsb = 16 * (qcw + 1);               // padded row stride in bytes
-  auto issue_q = [&]() {  // one load instruction per 64 chunks, spread over the waves
-    if (RD4_DEC_KNOBS && (a.dbg & 2048)) return;
-    for (int base = 64 * w; base < G * (qcw + 1); base += 64 * kWaves) {
-      const int idx = base + lane, r = idx / (qcw + 1), c = idx - r * (qcw + 1);
-      if (r < G && c < qcw) {
-        const uint8_t *src = (const uint8_t *)a.q +
-                             (((int64_t)tok * a.n_head + h0 + r) * kHD) * (a.q_f16 ? 2 : 4) + 16 * c;
-        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(q_lds + 16 * base), 16, 0, 0);
-      }
-    }
-  };
-  // int8 query path: wave w loads the rows it quantizes straight into registers
-  // (lane l: dims 4l..4l+3), ahead of its tile loads, so it waits for its own
-  // rows only, with no barrier and no LDS traffic
-  float xq[kI8 ? 8 / kWaves : 1][4];
-  auto load_q_own = [&]() {
-#pragma unroll
-    for (int m = 0; m < 8 / kWaves; ++m) {
-      const int r = w + kWaves * m;
-      const int64_t off = ((int64_t)tok * a.n_head + h0 + (r < G ? r : 0)) * kHD + 4 * lane;
-      if (a.q_f16) {
-        const uint2 hv = *(const uint2 *)((const uint16_t *)a.q + off);
-        xq[m][0] = h2f((uint16_t)hv.x);
-        xq[m][1] = h2f((uint16_t)(hv.x >> 16));
-        xq[m][2] = h2f((uint16_t)hv.y);
-        xq[m][3] = h2f((uint16_t)(hv.y >> 16));
-      } else {
-        const float4 fv = *(const float4 *)(a.q + off);
-        xq[m][0] = fv.x;
-        xq[m][1] = fv.y;
-        xq[m][2] = fv.z;
-        xq[m][3] = fv.w;
-      }
-    }
-  };
-  if (!pair) {
-    if constexpr (kI8) load_q_own();
-    else issue_q();
-  }
+  if constexpr (!pair && !kI8) issue_q();
 #ifndef RD4_DEC_PRE
 #define RD4_DEC_PRE 0
 #endif
