@@ -18,8 +18,8 @@
 //   * V block arrives the same way, same swizzle; the PV operand (16 dims x
 //     8 keys per lane group) is read straight out of it with the gfx950
 //     transposing LDS load (ds_read_b64_tr_b16), so no transpose pass;
-//   three K stages and two V stages: K two blocks ahead, V one, one CTA
-//   barrier per block;
+//   three K stages and two V stages: K two blocks ahead, V one, both requested
+//   after the block's QK^T phase, one CTA barrier per block;
 //   * S^T = K Q^T on v_mfma_f32_16x16x32_f16 (A = 16 keys x 32 dims of K from
 //     LDS, B = the wave's query rows in registers), O^T += V^T P^T likewise;
 //     in both phases a ring of operand fragments keeps several steps of LDS
@@ -81,9 +81,10 @@ constexpr int kPVD0 = RD4_PF_PVD;
 #define RD4_PF_QKD 4
 #endif
 constexpr int kQG = RD4_PF_QKG, kQD0 = RD4_PF_QKD;
-// the same at three waves per SIMD (12 waves per CTA)
+// the same at three waves per SIMD (12 waves per CTA): 3 / 3 steps 602 us, 4 / 3
+// 598, 4 / 4 597, 5 / 4 631 (spills) at 4096 queries over 8192 keys
 #ifndef RD4_PF_QKD_W12
-#define RD4_PF_QKD_W12 3
+#define RD4_PF_QKD_W12 4
 #endif
 #ifndef RD4_PF_PVD_W12
 #define RD4_PF_PVD_W12 3
@@ -101,14 +102,15 @@ constexpr int kQG = RD4_PF_QKG, kQD0 = RD4_PF_QKD;
 #ifndef RD4_PF_MASKBR
 #define RD4_PF_MASKBR 1
 #endif
-// where K(j + 2) is requested (0 at the top of block j, 1 after its QK^T phase,
-// 3 with V(j + 1) after it too)
 // K/V DMA by inline asm (1) or by the builtin (0)
 #ifndef RD4_PF_DMAASM
 #define RD4_PF_DMAASM 1
 #endif
+// where K(j + 2) is requested (0 at the top of block j, 1 after its QK^T phase,
+// 3 with V(j + 1) after it too). 4096 queries over 8192 keys, one run: 628 / 598 /
+// 594 us; 512 over 8192: 129 / 120 / 119.
 #ifndef RD4_PF_DMAPOS
-#define RD4_PF_DMAPOS 1
+#define RD4_PF_DMAPOS 3
 #endif
 // block max by max3 asm (1) or by fmaxf (0)
 #ifndef RD4_PF_SM
@@ -412,19 +414,17 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
   const int tr_kx = 4 * g + (n >> 2);                       // key & 15 of this source lane
   const int tr_off = tr_kx * (kHD * 2) + 8 * (n & 1);        // row and 8-byte half
   const int tr_m = 16 * ((n >> 1 & 1) ^ swz(tr_kx));        // swizzle term of the chunk
-  // lane offset of dim tile dt for dt = 0..7; tr_m < 256, so tile dt + 8 is
-  // the same offset + 256 (an instruction immediate)
-  int v_loff[8];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) v_loff[dt] = tr_off + ((32 * dt) ^ tr_m);
-  // LDS read offsets of the MFMA operands (block-invariant).
-  // K: key 16kt + n, dims 32b + 8g: slot (4b + g) ^ n = 4(b ^ (n>>2)) + (g ^ (n&3)).
-  int k_loff[8];
-#pragma unroll
-  for (int b = 0; b < 8; ++b) k_loff[b] = n * (kHD * 2) + 16 * ((4 * b + g) ^ swz(n));
+  // LDS read addresses of the MFMA operands in stage 0: the fragments differ in
+  // XORed bits (the stages are 512-byte aligned), so a block's addresses come from
+  // one register each, not from eight held offsets.
+  // V: dim tile dt: chunk term (32 dt) ^ tr_m for dt = 0..7; tr_m < 256, so tile
+  // dt + 8 is the same address + 256 (an instruction immediate).
+  // K: key 16kt + n, dims 32b + 8g: slot (4b + g) ^ swz(n).
+  auto lds_of = [](const uint8_t *x) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)x; };
+  const uint32_t v_at = lds_of(smem + kKStages * kKBytes) + tr_off + tr_m;
+  const uint32_t k_at = lds_of(smem) + n * (kHD * 2) + 16 * (g ^ swz(n));
 
-  // Issue order: K0 V0 K1, then in block j: V(j+1) at the top, K(j+2) after
-  // the QK^T phase.
+  // Issue order: K0 V0 K1, then in block j V(j+1) and K(j+2) after the QK^T phase.
   if (nbk > 0) {
     issue_k(b0, 0);
     issue_v(b0, 0);
@@ -454,14 +454,13 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
     __syncthreads();
 #endif
     const int ks2 = ks == 0 ? 2 : ks - 1;  // stage of K(blk + 2): (blk + 2) % 3
-    // DMA issue points (RD4_PF_DMAPOS, default 1): 0 both at the block top, 1 K(blk + 2)
+    // DMA issue points (RD4_PF_DMAPOS): 0 both at the block top, 1 K(blk + 2)
     // after the QK^T phase, 3 both after it
     if (!(RD4_PF_KNOB & 8)) {
       if (RD4_PF_DMAPOS != 3 && bi + 1 < nbk) issue_v(blk + 1, vs ^ 1);
       if (RD4_PF_DMAPOS == 0 && bi + 2 < nbk) issue_k(blk + 2, ks2);
     }
-    const uint8_t *kd = smem + ks * kKBytes;
-    const uint8_t *vd = smem + (kKStages + vs) * kKBytes;
+    const uint32_t k_st = k_at + ks * kKBytes, v_st = v_at + vs * kKBytes;
     ks = ks == 2 ? 0 : ks + 1;
     const int j0 = blk * kBN;
     const bool need_mask = (j0 + kBN - 1) > wave_min_lim;
@@ -481,7 +480,7 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
     u32x4 kr[kRing];
     auto read_kf = [&](int f) {
       kr[f % kRing] = (RD4_PF_KNOB & 1) ? __builtin_bit_cast(u32x4, qf[0][(f + 1) & 7])
-                                        : *(const lds_u32x4 *)(kd + (f >> 3) * 16 * (kHD * 2) + k_loff[f & 7]);
+                                        : *(lds_u32x4 *)((k_st ^ (64u * (f & 7))) + (f >> 3) * 16 * (kHD * 2));
       __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
@@ -504,7 +503,7 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
       const int kg = t >> 3, dt0 = 2 * (t & 7);
 #pragma unroll
       for (int d = 0; d < 2; ++d) {
-        const uint8_t *a0 = vd + v_loff[(dt0 + d) & 7] + (32 * kg) * (kHD * 2) + 256 * ((dt0 + d) >> 3);
+        const uint32_t a0 = (v_st ^ (32u * ((dt0 + d) & 7))) + (32 * kg) * (kHD * 2) + 256 * ((dt0 + d) >> 3);
         if (RD4_PF_KNOB & 2) {
           vb[buf][d] = qf[0][(dt0 + d) & 7];
           continue;
@@ -618,7 +617,7 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
     if (RD4_PF_PROBE & 2)
       __asm__ volatile(".rept 16\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\t.endr\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(pr_c) : "v"(qf[0][0]), "v"(qf[0][1]));
     if (RD4_PF_PROBE & 4)
-      __asm__ volatile(".rept 16\n\tds_read_b128 %0, %1\n\t.endr\n\ts_waitcnt lgkmcnt(0)" : "=v"(pr_d) : "v"((uint32_t)(uintptr_t)smem + k_loff[0]));
+      __asm__ volatile(".rept 16\n\tds_read_b128 %0, %1\n\t.endr\n\ts_waitcnt lgkmcnt(0)" : "=v"(pr_d) : "v"((uint32_t)(uintptr_t)smem + k_at));
 #endif
   }
 #if RD4_PF_PROBE
