@@ -219,9 +219,25 @@ __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int l
   const int r = conv_row(lane), b = conv_block(lane), key = key0 + r, sz = swz(key & 15);
   uint8_t *dst = hi_st + key * (kHD * 2);
   if constexpr (T == F16) {
+    bool nonfin = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      *(u32x4 *)(dst + 16 * ((4 * b + i) ^ sz)) = *(const u32x4 *)(raw + r * 512 + 64 * b + 16 * i);
+    for (int i = 0; i < 4; ++i) {
+      u32x4 x = *(const u32x4 *)(raw + r * 512 + 64 * b + 16 * i);
+      if (V) {  // values that are not finite enter as zeros (the kernel adds them for
+        // the rows that attend the key)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const bool lo = (x[c] & 0x7c00u) == 0x7c00u, hi = (x[c] & 0x7c000000u) == 0x7c000000u;
+          nonfin |= lo || hi;
+          x[c] &= (lo ? 0xffff0000u : 0xffffffffu) & (hi ? 0x0000ffffu : 0xffffffffu);
+        }
+      }
+      *(u32x4 *)(dst + 16 * ((4 * b + i) ^ sz)) = x;
+    }
+    if (V) {
+      const uint64_t nf = __ballot(nonfin);
+      if (b == 0) nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
+    }
   } else {
     uint32_t w[8], dm, ch[4], cl[4];
     block_words<T>(raw + r * (8 * block_bytes(T)), b, w, &dm);
@@ -595,14 +611,34 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
       convert_v(st ^ 1);
       refill();
     }
-    // V blocks that are not finite entered as zeros: remembered for the rows that
-    // attend their key
-    if (VLO) {
-      const uint8_t *nf = (const uint8_t *)(tb + 3 * kBN);
-      if (__any(nf[lane & 31] != 0))
+    // V values that are not finite entered as zeros. Of an f16 cache they are added
+    // here, for the rows that attend their key; blocks of a quantized one are
+    // remembered for those rows.
+    const uint8_t *nf = (const uint8_t *)(tb + 3 * kBN);
+    if (__any(nf[lane & 31] != 0)) {
 #pragma unroll 1
-        for (int key = 0; key < kBN; ++key)
+      for (int key = 0; key < kBN; ++key) {
+        if (nf[key] == 0 || j0 + key > kend) continue;  // (uniform; past kend a valid row was read again)
+        if constexpr (VLO) {
           if (j0 + key <= lim_row) poison |= nf[key];
+        } else {
+          float x = 0.0f;
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (16 * kt + i == (key & 0x13)) x = pf[kt][i];
+          x = __shfl(x, 4 * (key & 12) + n, 64) * (float)(1 << kPShift);
+          const uint16_t *vr = (const uint16_t *)(p.v + ((int64_t)(j0 + key) * p.n_head_kv + kvh) * (kHD * 2)) + 4 * g;
+#pragma unroll
+          for (int dt = 0; dt < 16; ++dt)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const uint16_t h = vr[16 * dt + c];
+              if ((h & 0x7c00u) == 0x7c00u && j0 + key <= lim_row) o[dt][c] = fmaf(x, h2f(h), o[dt][c]);
+            }
+        }
+      }
     }
   }
 

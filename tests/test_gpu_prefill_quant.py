@@ -122,3 +122,29 @@ def test_a_row_that_is_not_finite_stays_with_its_readers(rd4, orc, dev, which):
     hit[bad - pos0:, 6 * h:6 * h + 6, (slice(32 * b, 32 * b + 32) if which == "v" else slice(None))] = True
     assert np.array_equal(got[~hit], clean[~hit])
     assert not np.isfinite(got[hit]).any()
+
+
+def test_an_f16_v_value_that_is_not_finite_stays_with_its_readers(rd4, orc, dev):
+    """The same for single values of an f16 V cache beside a quantized K: the dims
+    that hold them are infinite or NaN from the key's row on, everything else as
+    without them."""
+    import torch
+    nh, nkv, pos0, nq, h = 24, 4, 40, 50, 2
+    n = pos0 + nq
+    k, v = rows_of(orc, 2, n, nkv, 1), rows_of(orc, 1, n, nkv, 2)
+    q = orc.randn(nq * nh * 256, 3).reshape(nq, nh, 256)
+    c = v.view(np.float16).reshape(n, nkv, 256)
+    for bad, d in ((47, 5), (63, 200), (64, 31), (75, 128)):
+        c[bad, h, d] = 0
+    clean, _ = run(rd4, torch, dev, q, k, v, pos0, nh, nkv, 2, 1)
+    hit = np.zeros(clean.shape, bool)
+    for bad, d, x in ((47, 5, np.inf), (63, 200, -np.inf), (64, 31, np.nan), (75, 128, np.inf)):
+        c[bad, h, d] = x
+        hit[bad - pos0:, 6 * h:6 * h + 6, d] = True
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=dev)
+    rd4.prefill(to_dev(q, torch, dev), to_dev(k, torch, dev), to_dev(v, torch, dev), out, pos0, nh, nkv, 256, 1 / 16,
+                2, 1)
+    got = out.cpu().numpy()
+    assert np.array_equal(got[~hit], clean[~hit])
+    assert not np.isfinite(got[hit]).any()
+    assert np.all(got[7:, 6 * h:6 * h + 6, 5] == np.inf)
