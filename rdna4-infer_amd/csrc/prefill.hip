@@ -28,19 +28,20 @@ int compute_units() {
 }
 
 // Rows per CTA and keys per block of a cache pair's MFMA kernel, and what a CTA
-// costs on an MI355X: us per key block (with up to half of the CUs busy, and
-// with all: the f16 kernel's blocks slow down with the clock), and us before and
-// after its blocks.
+// costs on an MI355X: us per key block, and us before and after its blocks. (The
+// f16 kernel's blocks take 2.2 us in a long call on few CUs and 3.2 on all; with a
+// few blocks each, first use and masks included, 3.4, and that is where the count
+// is close: 168 queries from position 0 take 32.1 us in one split, 26.9 in three.)
 struct Shape {
   int rows, keys;
-  double block_us, block_us_full, cta_us;
+  double block_us, cta_us;
 };
 Shape shape_of(int kt, int vt) {
-  if (kt == F16 && vt == F16) return {192, 64, 2.2, 3.2, 14.0};
-  return {128, 32, 3.0, 3.0, 14.0};
+  if (kt == F16 && vt == F16) return {192, 64, 3.4, 14.0};
+  return {128, 32, 3.0, 14.0};
 }
 // The merge launch: us of the launch, and bytes of records written and read per us.
-constexpr double kMergeUs = 3.0, kMergeBytesPerUs = 5e6;
+constexpr double kMergeUs = 2.0, kMergeBytesPerUs = 5e6;
 
 }  // namespace
 
@@ -79,16 +80,13 @@ int prefill_ksplits(const PrefillArgs &p, int kt, int vt, int64_t max_floats) {
     if (s > 1 && (blocks + per - 1) / per != s) continue;  // as many as a smaller count with the same blocks
     if (s > 1 && prefill_part_floats(p, s) > max_floats) break;
     const int64_t ctas = (int64_t)total * s;
-    const double busy = std::min(1.0, std::max(0.0, 2.0 * (double)ctas / cus - 1.0));
-    const double block_us = sh.block_us + (sh.block_us_full - sh.block_us) * busy;
-    const double one = per * block_us + sh.cta_us;
-    const double all = ((double)total * mean * block_us + (double)ctas * sh.cta_us) / cus;
+    const double one = per * sh.block_us + sh.cta_us;
+    const double all = ((double)total * mean * sh.block_us + (double)ctas * sh.cta_us) / cus;
     const double alike = std::min(1.0, std::max(0.0, 2.0 * mean / blocks - 0.5));
     const double even = std::max(one, all);
     double us = even + alike * std::max(0.0, (double)((ctas + cus - 1) / cus) * one - even);
     if (s > 1) us += kMergeUs + (double)prefill_part_floats(p, s) * 4 / kMergeBytesPerUs;
-    if (s == 1) best_us = 0.9 * us;  // (a split call is two launches: taken for a gain of a tenth or more)
-    else if (us < best_us) best = s, best_us = us;
+    if (s == 1 || us < best_us) best = s, best_us = us;
     if (ctas > 4 * cus) break;  // more only adds records
   }
   return best;
