@@ -639,7 +639,7 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
       float *rec = p.part + rr * kHD;
 #pragma unroll
       for (int dt = 0; dt < 16; ++dt)
-        if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[sl][dt];  // (m = -inf: the merge drops the record)
+        if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[sl][dt];  // (l = 0: the merge drops the record)
       if (g == 0) *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run[sl], L);
       continue;
     }
@@ -688,17 +688,21 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs p) {
       if (s0 + i < S) rv[i] = *(const floatx4 *)(rec + (int64_t)(s0 + i) * nr * kHD);
   };
   load(0);
+  // A split with no key of this row has l = 0 and counts for nothing, whatever its
+  // record holds. m = -inf alone does not say so: where every score of a split is
+  // NaN the running max stays at -inf and l is NaN, and the row must end as NaN.
+  const bool empty = r.y == 0.0f;
   const float M = wave_max(r.x);
-  const float wgt = (r.x == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(r.x - M);
-  const float L = wave_sum(r.x == -INFINITY ? 0.0f : wgt * r.y);
+  const float wgt = empty ? 0.0f : __builtin_amdgcn_exp2f(r.x - M);
+  const float L = wave_sum(empty ? 0.0f : wgt * r.y);
+  const uint64_t used = ~__ballot(empty);
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < S; s0 += kB) {
     if (s0) load(s0);
 #pragma unroll
     for (int i = 0; i < kB; ++i) {
       if (s0 + i >= S) break;
-      // (a split with no key of this row counts for nothing, whatever its record)
-      if (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r.x), s0 + i)) == -INFINITY) continue;
+      if (!((used >> (s0 + i)) & 1)) continue;
       const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wgt), s0 + i));
 #pragma unroll
       for (int c = 0; c < 4; ++c) acc[c] = fmaf(ws, rv[i][c], acc[c]);

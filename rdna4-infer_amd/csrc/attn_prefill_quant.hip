@@ -661,7 +661,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     float *rec = p.part + rr * kHD;
 #pragma unroll
     for (int dt = 0; dt < 16; ++dt)
-      if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[dt] * o_pw2;  // (m = -inf: the merge drops the record)
+      if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[dt] * o_pw2;  // (l = 0: the merge drops the record)
     if (g == 0) *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run, Ls);
     return;
   }

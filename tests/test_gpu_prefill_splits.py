@@ -33,3 +33,31 @@ def test_split_calls_match_oracle(rd4, orc, dev, t, nh, nkv, pos0, nq):
     if t != 1:
         want = np.asarray(want, np.float64).reshape(got[rows].shape)
         assert np.linalg.norm(got[rows] - want) <= 3e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("kt,vt", [(1, 1), (2, 2), (4, 5), (1, 2), (3, 1)])
+def test_a_split_whose_scores_are_all_nan_stays_nan(rd4, orc, dev, kt, vt):
+    """One K row that is NaN at the first key of a split (8 f16 or 15 quantized
+    one-block splits): the query at that position attends no other key of its
+    split, so the split's running max never leaves -inf. From the row on the head
+    is NaN, before it and in the other heads nothing changes."""
+    import torch
+    nh, nkv, pos0, nq, h = 24, 4, 400, 60, 1
+    n = pos0 + nq
+    k, v = orc.store_rows(kt, orc.randn(n * nkv * 256, 1)), orc.store_rows(vt, orc.randn(n * nkv * 256, 2))
+    q = to_dev(orc.randn(nq * nh * 256, 3).reshape(nq, nh, 256), torch, dev)
+
+    def run(kb):
+        out = torch.zeros(q.shape, dtype=torch.float32, device=dev)
+        rd4.prefill(q, to_dev(kb, torch, dev), to_dev(v, torch, dev), out, pos0, nh, nkv, 256, 1 / 16, kt, vt)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    clean = run(k)
+    for bad in (416, 447, 448):  # 448 starts a block of 32 and of 64 keys, 416 one of 32
+        kb = k.copy()
+        kb.view(np.uint8).reshape(n, nkv, -1)[bad, h, :2] = np.frombuffer(np.float16(np.nan).tobytes(), np.uint8)
+        got, hit = run(kb), np.zeros(clean.shape, bool)
+        hit[bad - pos0:, 6 * h:6 * h + 6] = True
+        assert np.isnan(got[hit]).all(), bad
+        assert np.array_equal(got[~hit], clean[~hit]), bad
