@@ -14,17 +14,23 @@
 //     comes to [1, 2)) and split: d * int has at most 19 significant bits, so
 //     K' = kh + kl exactly (blocks down to 2^-14 of the row's largest scale);
 //   * S = kl.qh + kh.ql + kh.qh, f32 accumulation, then times both powers of two;
-//   * p stays f32 for the row sum l; p * 2^(e - e0 + 7) (e the V row's power of
-//     two, e0 that of the CTA's first row) is split for O += vl.ph + vh.pl + vh.ph.
-//     The reference exponent of a row follows its largest s + e - e0, so the split
-//     value stays within 2^15 whatever the cache holds.
+//   * value rows are scaled by a power of two 2^e of the CTA (its block of 32 keys
+//     has its largest block scale between 1 and 2^8; a block that has not moves e,
+//     and O with it) and split like keys, exactly for blocks down to 2^-14;
+//   * p stays f32 for the row sum l; p * 2^7 is split for O += vl.ph + vh.pl + vh.ph:
+//     22 bits of a p down to 2^-10 of the row's largest, below that 2^-32 of the
+//     largest;
+//   * V blocks that this does not hold (scales further apart, or not finite) enter
+//     the products as zeros and are added in f32 for the rows that attend them.
 // f16 rows have no remainder part (and no scaling): two products instead of three.
 // Relative error against 64 bits, the VALU kernel (attn_generic.hip), which took
 // these calls before, in brackets, for q8_0: 1.2e-7 (1.3e-7) at 33 queries over 33
-// keys, 2.2e-7 (2.9e-7) over 233, 3.5e-7 (9.0e-7) over 8064. What it takes: the
+// keys, 2.1e-7 (2.6e-7) over 233, 3.5e-7 (8.8e-7) over 8064. What it takes: the
 // large products of S in four sums and the small ones in a fifth (one sum for
-// all: 2.0 times the error at 233 keys), the p split near 2^7 (near 1: 1.5 times),
-// and exp2 arguments near 0 for the largest p (e folded into them: 1.3 times).
+// all: 2.0 times the error at 233 keys), and the p split near 2^7 (near 1: 1.5
+// times). V's power of two is no part of p (a row's own exponent in p, as 2^e of it:
+// rows 2^17 smaller than another lost percents of what they add where the other's
+// dims are zero).
 //
 // Work decomposition: rows r = query * group + head of one kv head as in the
 // f16 kernel; CTA = 8 waves x 16 rows, 32-key blocks. Each wave owns 8 key rows of
@@ -66,9 +72,13 @@ constexpr int kW = 8;              // waves per CTA
 constexpr int kBM = 16 * kW;       // rows per CTA
 constexpr int kPart = kBN * kHD * 2;  // one f16 part of a block's K or V rows
 constexpr float kLog2e = 1.4426950408889634f;
-// the largest p * 2^(e - e0) of a row is kept between 2^kPShift and 2^(kPShift + 8):
-// terms 2^-14 of it still have normal f16 remainder parts
+// the largest p * 2^kPShift of a row is kept between 2^kPShift and 2^(kPShift + 8):
+// terms 2^-10 of it still have normal f16 remainder parts
 constexpr int kPShift = 7;
+// A V block's largest scale, as scaled, is kept between 2^0 and 2^(kVTop + 1)
+// (times 127 it is below f16's largest, and steps of the scales' exponents up to
+// kVMid either way leave e alone), placed at 2^kVMid when it is not.
+constexpr int kVTop = 7, kVMid = 4;
 
 // LDS: two stages of [K hi][K lo][V hi][V lo] (lo parts of quantized types
 // only), each wave's raw rows, then the per-key tables of both stages.
@@ -80,9 +90,10 @@ struct Lds {
   static constexpr int kRawK = KLO ? 3072 : 4096, kRawV = VLO ? 3072 : 4096;
   static constexpr int kRaw = 2 * kStage;
   static constexpr int kTab = kRaw + 4 * (kRawK + kRawV);
-  // per stage: f32 2^e of K rows, f32 2^(e - e0 + kPShift) and e - e0 of V rows,
-  // and one byte per V row with a bit for each of its blocks that is not finite
-  static constexpr int kTabStage = 3 * kBN * 4 + kBN;
+  // per stage: f32 2^e of K rows, one byte per V row with a bit for each of its
+  // blocks that is outside the products, and V's exponent e
+  static constexpr int kNf = kBN * 4, kE = kNf + kBN;
+  static constexpr int kTabStage = kE + 16;
   static constexpr int kBytes = kTab + 2 * kTabStage;
   static_assert(kBytes <= 160 * 1024, "LDS of a CU");
 };
@@ -111,6 +122,19 @@ __device__ __forceinline__ float max_groups4(float x) {
 // bank conflict (8 lanes per row in order: 2-way).
 __device__ __forceinline__ int conv_row(int lane) { return ((lane >> 4) & 1) | (((lane >> 2) & 3) << 1); }
 __device__ __forceinline__ int conv_block(int lane) { return (lane & 3) | ((lane >> 5) << 2); }
+// unsigned max over the wave
+__device__ __forceinline__ uint32_t max_wave_u32(uint32_t x) {
+  int v = (int)x;
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xF, 0xF, false));  // row_half_mirror
+  v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xF, 0xF, false));  // row_mirror
+  int a = v, b = v;
+  __asm__("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  a = max(a, b), b = a;
+  __asm__("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+  return __builtin_amdgcn_readfirstlane((uint32_t)max(a, b));
+}
 // unsigned max over the 8 lanes of a row
 __device__ __forceinline__ uint32_t max_row_u32(uint32_t x) {
   int v = (int)x;
@@ -203,19 +227,21 @@ __device__ __forceinline__ half2v block_pair(const uint32_t *w, int f) {
   }
 }
 
-// Exponent of a row's power of two, from the f16 magnitude bits of its blocks'
-// scales (one per lane of the row's 8; the largest finite one counts).
-__device__ __forceinline__ int row_exponent(uint32_t mag) {
-  return max((int)(max_row_u32(mag >= 0x7c00u ? 0u : mag) >> 10), 1) - 15;
+// Exponent of f16 magnitude bits (subnormals: that of the smallest normal), and the
+// larger finite magnitude of a block's scale d and, of q4_1, offset m (dm: d | m << 16).
+__device__ __forceinline__ int mag_exponent(uint32_t mag) { return max((int)(mag >> 10), 1) - 15; }
+__device__ __forceinline__ uint32_t finite_mag(uint32_t dm, bool with_m) {
+  const uint32_t d = dm & 0x7fffu, m = with_m ? (dm >> 16) & 0x7fffu : 0u;
+  return max(d >= 0x7c00u ? 0u : d, m >= 0x7c00u ? 0u : m);
 }
 
 // Convert the wave's 8 raw rows (lane: row conv_row, block conv_block; rb bytes per
 // row) into the stage rows at hi_st (their lo parts kPart bytes on) and the tables:
-// pw2_tab[key] = 2^(e - e0 + shift), and for V exp_tab[key] = e - e0 and
-// nf_tab[key] = the mask of blocks that are not finite.
+// for K pw2_tab[key] = 2^e, e the row's exponent; V comes with its exponent ev, and
+// nf_tab[key] = the mask of the row's blocks that are outside the products.
 template <int T, bool V>
 __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int lane, uint8_t *hi_st, float *pw2_tab,
-                                             float *exp_tab, uint8_t *nf_tab, int e0) {
+                                             uint8_t *nf_tab, int ev) {
   const int r = conv_row(lane), b = conv_block(lane), key = key0 + r, sz = swz(key & 15);
   uint8_t *dst = hi_st + key * (kHD * 2);
   if constexpr (T == F16) {
@@ -241,17 +267,21 @@ __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int l
   } else {
     uint32_t w[8], dm, ch[4], cl[4];
     block_words<T>(raw + r * (8 * block_bytes(T)), b, w, &dm);
-    // The row's power of two from its largest scale (q4_1: or offset) magnitude.
-    uint32_t mag = dm & 0x7fffu;
-    if (T == Q4_1) mag = max(mag, (dm >> 16) & 0x7fffu);
-    const bool nonfin = mag >= 0x7c00u;
-    const int e = row_exponent(mag);
+    // K: the row's power of two from its largest scale (q4_1: or offset) magnitude.
+    const int e = V ? ev : mag_exponent(max_row_u32(finite_mag(dm, T == Q4_1)));
     _Float16 d = __builtin_amdgcn_ldexph(__builtin_bit_cast(_Float16, (uint16_t)dm), -e);
     _Float16 m = T == Q4_1 ? __builtin_amdgcn_ldexph(__builtin_bit_cast(_Float16, (uint16_t)(dm >> 16)), -e) : (_Float16)0.0f;
-    // A block that is not finite: K keeps it (its keys' scores become NaN). V's
-    // enters the products as zeros, so that rows which do not attend the key keep
-    // their sums; nf_tab marks it, and the rows that attend the key end as NaN.
-    if (V && nonfin) d = (_Float16)0.0f, m = (_Float16)0.0f;
+    // A K block that is not finite stays (its keys' scores become NaN). A V block
+    // that is not finite, or whose scaled d or m falls below the normal f16 range
+    // and may lose bits, enters the products as zeros; nf_tab marks it.
+    bool out = false;
+    if (V) {
+      auto lost = [](uint32_t before, _Float16 x) {  // scaled: not normal, and not from a zero
+        return __builtin_amdgcn_classh(x, 0x2f7) && (before & 0x7fffu) != 0;
+      };
+      out = lost(dm, d) || (T == Q4_1 && lost(dm >> 16, m));
+      if (out) d = (_Float16)0.0f, m = (_Float16)0.0f;
+    }
 #pragma unroll
     for (int f = 0; f < 16; ++f) {
       const half2v q = block_pair<T>(w, f);
@@ -263,13 +293,10 @@ __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int l
         *(u32x4 *)(at + kPart) = u32x4{cl[0], cl[1], cl[2], cl[3]};
       }
     }
-    const uint64_t nf = __ballot(nonfin);
+    const uint64_t nf = __ballot(out);
     if (b == 0) {
-      pw2_tab[key] = __builtin_ldexpf(1.0f, V ? e - e0 + kPShift : e);
-      if (V) {
-        exp_tab[key] = (float)(e - e0);
-        nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
-      }
+      if (V) nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
+      else pw2_tab[key] = __builtin_ldexpf(1.0f, e);
     }
   }
 }
@@ -342,32 +369,51 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     const int c = min(64 * i + lane, 8 * nch - 1);  // (surplus lanes repeat the last chunk into the padding)
     c_at[i] = (uint32_t)(8 * (w & 3) + c / nch) << 16 | (uint32_t)(16 * (c % nch));
   }
+  // V waves: scale (q4_1: and offset) of 4 of a block's 256 (key, 32 dims) pairs,
+  // loaded beside its rows: each V wave needs the exponent of all 32 keys before it
+  // converts its own 8
+  uint32_t v_dm[4];
+  int e_v = 0;
   auto issue = [&](int bi) RD4_INLINE {
     const int j0 = (b0 + bi) * kBN;
+    if (VLO && isv) {
+      const uint8_t *at = my_base + (int64_t)j0 * my_stride + (lane & 7) * (rb >> 3);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint8_t *x = at + (int64_t)min(8 * i + (lane >> 3), kend - j0) * my_stride;
+        if (VT == Q4_1 || (VT < 0 && VFULL)) v_dm[i] = *(const uint32_t *)x;
+        else v_dm[i] = ld_u16(x);
+      }
+    }
     const uint8_t *src = uniform_ptr(my_base + (int64_t)j0 * my_stride);
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // keys past kend re-read a valid row (masked later)
       if (i < n_dma) dma16(src, (uint32_t)(min((int)(c_at[i] >> 16), kend - j0) * my_stride) + (c_at[i] & 0xffffu), lds_addr(raw + 1024 * i));
   };
-  // O and p * 2^e are kept relative to the exponent of the CTA's first V row, so
-  // that p itself is near 1 where it matters (the argument of its exp2 near 0)
-  int e0 = 0;
-  if (VLO && nbk > 0) {
-    const int vrb = (int)row_bytes(p.vt, kHD);
-    const uint8_t *blk = p.v + ((int64_t)b0 * kBN * p.n_head_kv + kvh) * vrb + conv_block(lane) * (vrb >> 3);
-    uint32_t mag = ld_u16(blk) & 0x7fffu;
-    if (p.vt == Q4_1) mag = max(mag, (uint32_t)ld_u16(blk + 2) & 0x7fffu);
-    e0 = __builtin_amdgcn_readfirstlane(row_exponent(mag));
-  }
   auto tab = [&](int st) RD4_INLINE { return (float *)(smem + L::kTab + st * L::kTabStage); };
   auto convert_as = [&](auto type, auto is_v, int st) RD4_INLINE {
     float *t = tab(st);
     uint8_t *sb = smem + st * L::kStage;
     constexpr int T = decltype(type)::value;
-    if constexpr (decltype(is_v)::value)
-      convert_rows<T, true>(raw, 8 * (w & 3), lane, sb + L::VH, t + kBN, t + 2 * kBN, (uint8_t *)(t + 3 * kBN), e0);
-    else
-      convert_rows<T, false>(raw, 8 * (w & 3), lane, sb + L::KH, t, nullptr, nullptr, 0);
+    if constexpr (decltype(is_v)::value) {
+      if (VLO) {  // e_v: the same in the four V waves
+        uint32_t mag = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mag = max(mag, max(v_dm[i] & 0x7fffu, T == Q4_1 ? (v_dm[i] >> 16) & 0x7fffu : 0u));
+        mag = max_wave_u32(mag);
+        if (mag >= 0x7c00u) {  // (uniform) the largest finite one counts
+          mag = 0;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mag = max(mag, finite_mag(v_dm[i], T == Q4_1));
+          mag = max_wave_u32(mag);
+        }
+        const int top = mag_exponent(mag) - e_v;
+        if (mag && (top < 0 || top > kVTop)) e_v += top - kVMid;
+        if (w == 4 && lane == 0) *(int *)((uint8_t *)t + L::kE) = e_v;
+      }
+      convert_rows<T, true>(raw, 8 * (w & 3), lane, sb + L::VH, nullptr, (uint8_t *)t + L::kNf, e_v);
+    } else
+      convert_rows<T, false>(raw, 8 * (w & 3), lane, sb + L::KH, t, nullptr, 0);
   };
   // this wave's rows into stage st: K for waves 0-3, V for 4-7
   auto convert_k = [&](int st) RD4_INLINE {
@@ -450,7 +496,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
 #pragma unroll
   for (int i = 0; i < 16; ++i) o[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.0f;
-  uint32_t poison = 0;  // 32-dim blocks of this row that met a V block which is not finite
+  int e_o = 0;  // O is in units of 2^(e_o - kPShift)
 
   // transposing V reads (as in the f16 kernel): source lane s of a 16-lane group
   // points at key 4g + s/4, dims 4(s%4)..+3 of a 16-dim tile
@@ -476,16 +522,19 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   for (int bi = 0; bi < nbk; ++bi) {
     const int st = bi & 1;
     const int j0 = (b0 + bi) * kBN;
-    // this wave's raw rows of block bi + 1 have landed, and its conversion of
-    // block bi is written; past the barrier so is every wave's, and all are done
-    // reading the other stage
-    __asm__ volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // this wave's conversion of block bi is written; past the barrier so is every
+    // wave's, and all are done reading the other stage. (Raw rows are waited for by
+    // the wave that converts them: K's here, V's, which were requested a moment
+    // ago, after the products.)
+    __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const bool more = bi + 1 < nbk;
+    auto landed = [&]() RD4_INLINE { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
     auto refill = [&]() RD4_INLINE {
       __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // raw rows read before they are overwritten
       if (bi + 2 < nbk) issue(bi + 2);
     };
     if (more && !isv) {
+      landed();
       convert_k(st ^ 1);
       refill();
     }
@@ -526,21 +575,19 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
       }
     }
     // ---- online softmax: lane = row n, keys 16 kt + 4 g + i. The running max
-    // (m_run, in log2) follows s + e (e: the V row's exponent), which bounds p * 2^e.
+    // (m_run, in log2) follows s, to within 8.
     half8 ph, pl;
     float pf[2][4];
+    const uint8_t *nf = (const uint8_t *)tb + L::kNf;
+    const uint32_t nf_lane = nf[lane & 31];  // (read here, used after the products)
+    const int e_st = VLO ? *(const int *)((const uint8_t *)tb + L::kE) : 0;
     {
-      floatx4 vp[2], ve[2];
+      if (KLO) {
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        if (KLO) {
+        for (int kt = 0; kt < 2; ++kt) {
           const floatx4 ks = *(const floatx4 *)(tb + 16 * kt + 4 * g);
 #pragma unroll
           for (int i = 0; i < 4; ++i) s[kt][i] *= ks[i];
-        }
-        if (VLO) {
-          vp[kt] = *(const floatx4 *)(tb + kBN + 16 * kt + 4 * g);
-          ve[kt] = *(const floatx4 *)(tb + 2 * kBN + 16 * kt + 4 * g);
         }
       }
       if (j0 + kBN - 1 > wave_min_lim) {  // wave-uniform
@@ -554,7 +601,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, VLO ? fmaf(s[kt][i], c_row, ve[kt][i]) : s[kt][i] * c_row);
+        for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[kt][i] * c_row);
       tmax = max_groups4(tmax);
       const bool bump = tmax > m_run + 8.0f;
       if (__any(bump)) {
@@ -572,7 +619,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
         for (int i = 0; i < 4; ++i) {
           const float pv = __builtin_amdgcn_exp2f(fmaf(s[kt][i], c_row, -m_use));
           pf[kt][i] = pv;
-          const float pp = pv * (VLO ? vp[kt][i] : (float)(1 << kPShift));
+          const float pp = pv * (float)(1 << kPShift);
           const _Float16 h = (_Float16)pp;
           ph[4 * kt + i] = h;
           pl[4 * kt + i] = (_Float16)(pp - (float)h);
@@ -581,6 +628,15 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     }
 
     // ---- O^T += V^T P^T: 16 dim tiles, two transposing loads per operand
+    if (VLO) {
+      const int e = __builtin_amdgcn_readfirstlane(e_st);
+      if (e != e_o) {  // (uniform)
+        const float f = __builtin_ldexpf(1.0f, e_o - e);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[i] *= f;
+        e_o = e;
+      }
+    }
     {
       constexpr int D = kRing;
       half8 fh[D], fl[D];
@@ -608,44 +664,47 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
       }
     }
     if (more && isv) {
+      landed();
       convert_v(st ^ 1);
       refill();
     }
-    // V values that are not finite entered as zeros. Of an f16 cache they are added
-    // here, for the rows that attend their key; blocks of a quantized one are
-    // remembered for those rows.
-    const uint8_t *nf = (const uint8_t *)(tb + 3 * kBN);
-    if (__any(nf[lane & 31] != 0)) {
+    // What entered as zeros (f16 values that are not finite, blocks of a quantized
+    // cache outside the scaled range) is added here, for the rows that attend the key.
+    if (__any(nf_lane != 0)) {
+      const int v_rb = (int)row_bytes(p.vt, kHD), v_stride = p.n_head_kv * v_rb;
+      auto load_v = [&](const uint8_t *vr, int d, float v[4]) RD4_INLINE {
+        if constexpr (VT >= 0) load4<VT>(vr, d, v);
+        else if constexpr (VFULL) load4<Q4_1>(vr, d, v);
+        else if (p.vt == Q8_0) load4<Q8_0>(vr, d, v);
+        else if (p.vt == Q4_0) load4<Q4_0>(vr, d, v);
+        else load4<Q5_0>(vr, d, v);
+      };
 #pragma unroll 1
       for (int key = 0; key < kBN; ++key) {
-        if (nf[key] == 0 || j0 + key > kend) continue;  // (uniform; past kend a valid row was read again)
-        if constexpr (VLO) {
-          if (j0 + key <= lim_row) poison |= nf[key];
-        } else {
-          float x = 0.0f;
+        const uint32_t blocks = __builtin_amdgcn_readfirstlane((uint32_t)nf[key]);
+        if (blocks == 0 || j0 + key > kend) continue;  // (past kend a valid row was read again)
+        float x = 0.0f;
 #pragma unroll
-          for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (16 * kt + i == (key & 0x13)) x = pf[kt][i];
-          x = __shfl(x, 4 * (key & 12) + n, 64) * (float)(1 << kPShift);
-          const uint16_t *vr = (const uint16_t *)(p.v + ((int64_t)(j0 + key) * p.n_head_kv + kvh) * (kHD * 2)) + 4 * g;
+          for (int i = 0; i < 4; ++i)
+            if (16 * kt + i == (key & 0x13)) x = pf[kt][i];
+        x = __builtin_ldexpf(__shfl(x, 4 * (key & 12) + n, 64), kPShift - e_o);
+        const uint8_t *vr = p.v + (int64_t)(j0 + key) * v_stride + (int64_t)kvh * v_rb;
+        const bool on = j0 + key <= lim_row;
 #pragma unroll
-          for (int dt = 0; dt < 16; ++dt)
+        for (int dt = 0; dt < 16; ++dt) {
+          if (!((blocks >> (dt >> 1)) & 1)) continue;  // (uniform)
+          int g4 = 4 * g;
+          __asm__ volatile("" : "+v"(g4)::"memory");  // (one tile's addresses at a time: all together spill)
+          float v[4];
+          load_v(vr, 16 * dt + g4, v);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const uint16_t h = vr[16 * dt + c];
-              if ((h & 0x7c00u) == 0x7c00u && j0 + key <= lim_row) o[dt][c] = fmaf(x, h2f(h), o[dt][c]);
-            }
+          for (int c = 0; c < 4; ++c)
+            if (on && (VLO || !(fabsf(v[c]) < INFINITY))) o[dt][c] = fmaf(x, v[c], o[dt][c]);
         }
       }
     }
-  }
-
-  if (VLO && __any(poison != 0)) {
-#pragma unroll
-    for (int dt = 0; dt < 16; ++dt)
-      if ((poison >> (dt >> 1)) & 1) o[dt] = floatx4{NAN, NAN, NAN, NAN};
   }
 
   // ---- epilogue: l over the 4 key groups, then the record of a key split, or
@@ -655,7 +714,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   Ls += __shfl_xor(Ls, 32, 64);
   if (row >= n_rows) return;
   const int q = row / grp, head = kvh * grp + row % grp;
-  const float o_pw2 = __builtin_ldexpf(1.0f, e0 - kPShift);
+  const float o_pw2 = __builtin_ldexpf(1.0f, e_o - kPShift);
   if (p.n_ksplit > 1) {
     const int64_t nr = (int64_t)p.n_q * p.n_head, rr = (int64_t)ksp * nr + (int64_t)q * p.n_head + head;
     float *rec = p.part + rr * kHD;
