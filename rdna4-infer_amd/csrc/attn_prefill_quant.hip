@@ -11,9 +11,11 @@
 //   * a query row is scaled by a power of two (its largest |q * scale * log2e|
 //     comes to [2^8, 2^9)) and split, q' = qh + ql to 2^-22 of the row's largest;
 //   * a quantized key row is scaled by a power of two (its largest block scale
-//     comes to [1, 2)) and split: d * int has at most 19 significant bits, so
-//     K' = kh + kl exactly (blocks down to 2^-14 of the row's largest scale);
+//     comes to [2^7, 2^8)) and split: d * int has at most 19 significant bits, so
+//     K' = kh + kl exactly (blocks down to 2^-21 of the row's largest scale);
 //   * S = kl.qh + kh.ql + kh.qh, f32 accumulation, then times both powers of two;
+//     the scores of a key row that this does not hold (scales further apart, values
+//     that are not finite) are formed in f32 from the row itself;
 //   * value rows are scaled by a power of two 2^e of the CTA (its block of 32 keys
 //     has its largest block scale between 1 and 2^8; a block that has not moves e,
 //     and O with it) and split like keys, exactly for blocks down to 2^-14;
@@ -79,6 +81,7 @@ constexpr int kPShift = 7;
 // (times 127 it is below f16's largest, and steps of the scales' exponents up to
 // kVMid either way leave e alone), placed at 2^kVMid when it is not.
 constexpr int kVTop = 7, kVMid = 4;
+constexpr int kKTop = 7;  // a K row's largest scale, as scaled, is in [2^kKTop, 2^(kKTop + 1))
 
 // LDS: two stages of [K hi][K lo][V hi][V lo] (lo parts of quantized types
 // only), each wave's raw rows, then the per-key tables of both stages.
@@ -91,8 +94,8 @@ struct Lds {
   static constexpr int kRaw = 2 * kStage;
   static constexpr int kTab = kRaw + 4 * (kRawK + kRawV);
   // per stage: f32 2^e of K rows, one byte per V row with a bit for each of its
-  // blocks that is outside the products, and V's exponent e
-  static constexpr int kNf = kBN * 4, kE = kNf + kBN;
+  // blocks that is outside the products, the same per K row, and V's exponent e
+  static constexpr int kNf = kBN * 4, kKm = kNf + kBN, kE = kKm + kBN;
   static constexpr int kTabStage = kE + 16;
   static constexpr int kBytes = kTab + 2 * kTabStage;
   static_assert(kBytes <= 160 * 1024, "LDS of a CU");
@@ -237,51 +240,43 @@ __device__ __forceinline__ uint32_t finite_mag(uint32_t dm, bool with_m) {
 
 // Convert the wave's 8 raw rows (lane: row conv_row, block conv_block; rb bytes per
 // row) into the stage rows at hi_st (their lo parts kPart bytes on) and the tables:
-// for K pw2_tab[key] = 2^e, e the row's exponent; V comes with its exponent ev, and
-// nf_tab[key] = the mask of the row's blocks that are outside the products.
+// for K pw2_tab[key] = 2^e, e the row's exponent; V comes with its exponent ev.
+// nf_tab[key] = the mask of the row's blocks that are outside the products: V's are
+// zeros in the stage, a K row with any is left to the f32 path as a whole.
 template <int T, bool V>
 __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int lane, uint8_t *hi_st, float *pw2_tab,
                                              uint8_t *nf_tab, int ev) {
   const int r = conv_row(lane), b = conv_block(lane), key = key0 + r, sz = swz(key & 15);
   uint8_t *dst = hi_st + key * (kHD * 2);
+  bool out = false;
   if constexpr (T == F16) {
     bool nonfin = false;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       u32x4 x = *(const u32x4 *)(raw + r * 512 + 64 * b + 16 * i);
-      if (V) {  // values that are not finite enter as zeros (the kernel adds them for
-        // the rows that attend the key)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const bool lo = (x[c] & 0x7c00u) == 0x7c00u, hi = (x[c] & 0x7c000000u) == 0x7c000000u;
-          nonfin |= lo || hi;
-          x[c] &= (lo ? 0xffff0000u : 0xffffffffu) & (hi ? 0x0000ffffu : 0xffffffffu);
-        }
+      for (int c = 0; c < 4; ++c) {
+        const bool lo = (x[c] & 0x7c00u) == 0x7c00u, hi = (x[c] & 0x7c000000u) == 0x7c000000u;
+        nonfin |= lo || hi;
+        if (V) x[c] &= (lo ? 0xffff0000u : 0xffffffffu) & (hi ? 0x0000ffffu : 0xffffffffu);
       }
       *(u32x4 *)(dst + 16 * ((4 * b + i) ^ sz)) = x;
     }
-    if (V) {
-      const uint64_t nf = __ballot(nonfin);
-      if (b == 0) nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
-    }
+    out = nonfin;
   } else {
     uint32_t w[8], dm, ch[4], cl[4];
     block_words<T>(raw + r * (8 * block_bytes(T)), b, w, &dm);
     // K: the row's power of two from its largest scale (q4_1: or offset) magnitude.
-    const int e = V ? ev : mag_exponent(max_row_u32(finite_mag(dm, T == Q4_1)));
+    const int e = V ? ev : mag_exponent(max_row_u32(finite_mag(dm, T == Q4_1))) - kKTop;
     _Float16 d = __builtin_amdgcn_ldexph(__builtin_bit_cast(_Float16, (uint16_t)dm), -e);
     _Float16 m = T == Q4_1 ? __builtin_amdgcn_ldexph(__builtin_bit_cast(_Float16, (uint16_t)(dm >> 16)), -e) : (_Float16)0.0f;
-    // A K block that is not finite stays (its keys' scores become NaN). A V block
-    // that is not finite, or whose scaled d or m falls below the normal f16 range
-    // and may lose bits, enters the products as zeros; nf_tab marks it.
-    bool out = false;
-    if (V) {
-      auto lost = [](uint32_t before, _Float16 x) {  // scaled: not normal, and not from a zero
-        return __builtin_amdgcn_classh(x, 0x2f7) && (before & 0x7fffu) != 0;
-      };
-      out = lost(dm, d) || (T == Q4_1 && lost(dm >> 16, m));
-      if (out) d = (_Float16)0.0f, m = (_Float16)0.0f;
-    }
+    // outside: not finite, or d or m, as scaled, below the normal f16 range, where it
+    // may lose bits
+    auto lost = [](uint32_t before, _Float16 x) {  // scaled: not normal, and not from a zero
+      return __builtin_amdgcn_classh(x, 0x2f7) && (before & 0x7fffu) != 0;
+    };
+    out = lost(dm, d) || (T == Q4_1 && lost(dm >> 16, m));
+    if (V && out) d = (_Float16)0.0f, m = (_Float16)0.0f;
 #pragma unroll
     for (int f = 0; f < 16; ++f) {
       const half2v q = block_pair<T>(w, f);
@@ -293,12 +288,10 @@ __device__ __forceinline__ void convert_rows(const uint8_t *raw, int key0, int l
         *(u32x4 *)(at + kPart) = u32x4{cl[0], cl[1], cl[2], cl[3]};
       }
     }
-    const uint64_t nf = __ballot(out);
-    if (b == 0) {
-      if (V) nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
-      else pw2_tab[key] = __builtin_ldexpf(1.0f, e);
-    }
+    if (!V && b == 0) pw2_tab[key] = __builtin_ldexpf(1.0f, e);
   }
+  const uint64_t nf = __ballot(out);
+  if (b == 0) nf_tab[key] = (uint8_t)(((nf >> (lane & 0x1c)) & 15u) | (((nf >> ((lane & 0x1c) + 32)) & 15u) << 4));
 }
 
 }  // namespace
@@ -413,7 +406,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
       }
       convert_rows<T, true>(raw, 8 * (w & 3), lane, sb + L::VH, nullptr, (uint8_t *)t + L::kNf, e_v);
     } else
-      convert_rows<T, false>(raw, 8 * (w & 3), lane, sb + L::KH, t, nullptr, 0);
+      convert_rows<T, false>(raw, 8 * (w & 3), lane, sb + L::KH, t, (uint8_t *)t + L::kKm, 0);
   };
   // this wave's rows into stage st: K for waves 0-3, V for 4-7
   auto convert_k = [&](int st) RD4_INLINE {
@@ -545,6 +538,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     // (The small products go to a sum of their own and the large ones to four, so
     // that few roundings happen at the size of the whole sum.)
     floatx4 s[2];
+    const uint32_t km_lane = ((const uint8_t *)tb + L::kKm)[lane & 31];
     {
       constexpr int D = kRing;
       u32x4 fh[D], fl[D];
@@ -588,6 +582,46 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
           const floatx4 ks = *(const floatx4 *)(tb + 16 * kt + 4 * g);
 #pragma unroll
           for (int i = 0; i < 4; ++i) s[kt][i] *= ks[i];
+        }
+      }
+      // K rows outside the products: their scores in f32 from the cache
+      const uint32_t out_keys = (uint32_t)__ballot(km_lane != 0);
+      if (out_keys) {
+        const int k_rb = (int)row_bytes(p.kt, kHD), k_stride = p.n_head_kv * k_rb;
+        auto load_k = [&](const uint8_t *kr, int d, float v[4]) RD4_INLINE {
+          if constexpr (KT >= 0) load4<KT>(kr, d, v);
+          else if constexpr (!KLO) load4<F16>(kr, d, v);
+          else if (p.kt == Q8_0) load4<Q8_0>(kr, d, v);
+          else if (p.kt == Q4_0) load4<Q4_0>(kr, d, v);
+          else if (p.kt == Q5_0) load4<Q5_0>(kr, d, v);
+          else load4<Q4_1>(kr, d, v);
+        };
+        int rr = min(row, n_rows - 1), gg = g;
+        __asm__ volatile("" : "+v"(rr), "+v"(gg));  // (addresses formed here, not held through the loop)
+        const int64_t qat = ((int64_t)(rr / grp) * p.n_head + kvh * grp + rr % grp) * kHD;
+        const float sl2 = p.scale * kLog2e, up = 1.0f / c_row;  // (up: a power of two)
+#pragma unroll 1
+        for (int key = 0; key < kBN; ++key) {
+          if (!((out_keys >> key) & 1) || j0 + key > kend) continue;  // (past kend a valid row was read again)
+          const uint8_t *kr = p.k + (int64_t)(j0 + key) * k_stride + (int64_t)kvh * k_rb;
+          float dot = 0.0f;
+#pragma unroll 1
+          for (int d0 = 0; d0 < kHD; d0 += 16) {
+            const int d = d0 + 4 * gg;
+            float kv[4], qv[4];
+            load_k(kr, d, kv);
+            if (p.q_f16) load4<F16>((const uint8_t *)p.q + 2 * qat, d, qv);
+            else load4<F32>((const uint8_t *)p.q + 4 * qat, d, qv);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) dot = fmaf(qv[c] * sl2 * up, kv[c], dot);
+          }
+          dot += __shfl_xor(dot, 16, 64);
+          dot += __shfl_xor(dot, 32, 64);
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (16 * kt + i == (key & 0x13) && g == ((key >> 2) & 3)) s[kt][i] = dot;
         }
       }
       if (j0 + kBN - 1 > wave_min_lim) {  // wave-uniform

@@ -1,5 +1,5 @@
-"""Prefill over quantized caches where V values lie far apart (blocks of one row,
-whole rows) or are not finite. The path
+"""Prefill over quantized caches where values lie far apart: blocks of one V row,
+blocks of one K row, and values that are not finite. The path
 holds its operands as f16 pairs; what such a pair cannot hold takes an f32 path, so
 the results keep the tolerance of the path's other tests (3e-6, there derived), here
 for each 32-dim block of the output by itself, and are infinite or NaN where the
@@ -62,6 +62,24 @@ def test_v_blocks_far_apart(rd4, orc, dev, kt, vt, bits, how):
     assert err <= REL, err
 
 
+@pytest.mark.parametrize("kt,vt", [(2, 2), (3, 3), (4, 5), (5, 1)])
+@pytest.mark.parametrize("bits", [15, 19, 23, 26])
+def test_k_blocks_far_apart(rd4, orc, dev, kt, vt, bits):
+    """K's block 5 is 2^bits of the others; the queries are zero there (the scores
+    come from the small blocks alone)."""
+    import torch
+    pos0, nq = 90, 40
+    n = pos0 + nq
+    x = orc.randn(n * NKV * HD, 1).reshape(n, NKV, 8, 32) * np.float32(2000 * 2.0 ** -bits)
+    x[:, :, 5] *= np.float32(2.0 ** bits)
+    q = orc.randn(nq * NH * HD, 3).reshape(nq, NH, 8, 32) * np.float32(2.0 ** bits / 2000)
+    q[:, :, 5] = 0
+    q = q.reshape(nq, NH, HD)
+    k, v = orc.store_rows(kt, x.ravel()), orc.store_rows(vt, orc.randn(n * NKV * HD, 2))
+    err = block_error(run(rd4, torch, dev, q, k, v, pos0, kt, vt), oracle(orc, q, k, v, pos0, kt, vt))
+    assert err <= REL, err
+
+
 def like_valu(rd4, torch, dev, monkeypatch, q, k, v, pos0, kt, vt):
     """The call on the matrix cores and in the VALU kernel: infinite and NaN in the
     same places, and as close elsewhere as two f32 results are."""
@@ -74,6 +92,33 @@ def like_valu(rd4, torch, dev, monkeypatch, q, k, v, pos0, kt, vt):
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     assert np.linalg.norm(got[fin] - want[fin]) <= 2 * REL * np.linalg.norm(want[fin])
     return want
+
+
+@pytest.mark.parametrize("kt,vt", [(1, 2), (1, 5), (2, 2), (4, 5), (3, 1)])
+@pytest.mark.parametrize("sign", [-1.0, 1.0])
+def test_infinite_k(rd4, orc, dev, monkeypatch, kt, vt, sign):
+    """K rows with an infinite value (f16) or an infinite block scale over values of
+    one sign: scores of -inf leave the key out, +inf make the head NaN."""
+    import torch
+    pos0, nq, h = 60, 40, 2
+    n = pos0 + nq
+    x = orc.randn(n * NKV * HD, 1).reshape(n, NKV, HD)
+    x[:, :, 64:96] = 0.5 + np.abs(x[:, :, 64:96])
+    q = orc.randn(nq * NH * HD, 3).reshape(nq, NH, HD)
+    q[:, :, 64:96] = 0.1 + np.abs(q[:, :, 64:96])
+    k, v = orc.store_rows(kt, x.ravel()), orc.store_rows(vt, orc.randn(n * NKV * HD, 2))
+    # (q4_0 / q5_0 store d < 0 with levels below the offset where the largest value is
+    # positive; q4_1 as d and m)
+    rows = k.view(np.uint8).reshape(n, NKV, -1)
+    for r in (0, 7, 61, 64, 95):
+        if kt == 1:
+            rows.view(np.float16)[r, h, 70] = sign * np.inf
+        else:
+            b = rows[r, h].reshape(8, -1)[2]
+            d = b[:2].view(np.float16)
+            d[0] = np.copysign(np.inf, sign * float(d[0]))
+    want = like_valu(rd4, torch, dev, monkeypatch, q, k, v, pos0, kt, vt)
+    assert np.isfinite(want[:, 6 * h + 6:]).all() and (kt != 1 or np.isfinite(want).all() == (sign < 0))
 
 
 @pytest.mark.parametrize("kt,vt", [(2, 2), (3, 3), (1, 5), (5, 4), (2, 1)])
