@@ -9,7 +9,9 @@
 // Precision: 32-bit, on f16 matrix instructions. Every operand enters as an
 // f16 hi part plus the f16 remainder:
 //   * a query row is scaled by a power of two (its largest |q * scale * log2e|
-//     comes to [2^8, 2^9)) and split, q' = qh + ql to 2^-22 of the row's largest;
+//     comes to [2^8, 2^9)) and split, q' = qh + ql: 22 bits of a value down to 2^-10
+//     of the row's largest, below that 2^-34 of the largest. Rows with 8 consecutive
+//     dims all below 2^-10 (and not zero), or with an infinity, take f32 scores;
 //   * a quantized key row is scaled by a power of two (its largest block scale
 //     comes to [2^7, 2^8)) and split: d * int has at most 19 significant bits, so
 //     K' = kh + kl exactly (blocks down to 2^-21 of the row's largest scale);
@@ -165,6 +167,22 @@ __device__ __forceinline__ const uint8_t *uniform_ptr(const uint8_t *ptr) {
   return (const uint8_t *)(((uint64_t)hi << 32) | lo);
 }
 
+// The kernel's arguments read again where they are used (the f32 paths), and a
+// pointer among them: held in scalar registers through the loop they spill (12 of
+// them, read back in each block: 338 -> 347 us at 512 queries over 8192 keys).
+__device__ __forceinline__ PrefillArgs args_again() {
+  const __attribute__((address_space(4))) PrefillArgs *a =
+      (const __attribute__((address_space(4))) PrefillArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  __asm__ volatile("" : "+s"(a));
+  PrefillArgs r;
+  __builtin_memcpy(&r, (const PrefillArgs *)a, sizeof(r));
+  return r;
+}
+template <typename T>
+__device__ __forceinline__ const T *global_ptr(const T *x) {
+  return (const T *)(const __attribute__((address_space(1))) T *)x;
+}
+
 // Two integers as an f16 pair times the block scale -> hi pair and exact
 // remainder pair (an f16 product's rounding error is itself an f16).
 __device__ __forceinline__ void split_mul(half2v q, half2v d, uint32_t &hi, uint32_t &lo) {
@@ -229,6 +247,36 @@ __device__ __forceinline__ half2v block_pair(const uint32_t *w, int f) {
     return as_h2(n | 0x64006400u) + c;
   }
 }
+
+// 32-dim block b of a cache row as block_words reads it (f16: its values), and the
+// values 4 c .. 4 c + 3 of it.
+template <int T>
+struct RowBlock {
+  uint32_t w[T == F16 ? 16 : 8], dm;
+  __device__ __forceinline__ void read(const uint8_t *row, int b) {
+    if constexpr (T == F16) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) *(u32x4 *)(w + 4 * i) = *(const u32x4 *)(row + 64 * b + 16 * i);
+    } else {
+      block_words<T>(row, b, w, &dm);
+    }
+  }
+  __device__ __forceinline__ void values(int c, float v[4]) const {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      half2v q;
+      if constexpr (T == F16) q = as_h2(w[2 * c + i]);
+      else q = block_pair<T>(w, 2 * c + i);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        float x = (float)q[e];
+        if constexpr (T != F16) x = mul_rn(h2f((uint16_t)dm), x);
+        if constexpr (T == Q4_1) x = add_rn(x, h2f((uint16_t)(dm >> 16)));
+        v[2 * i + e] = x;
+      }
+    }
+  }
+};
 
 // Exponent of f16 magnitude bits (subnormals: that of the smallest normal), and the
 // larger finite magnitude of a block's scale d and, of q4_1, offset m (dm: d | m << 16).
@@ -436,6 +484,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   const int lim_row = limit_of(row);
   half8 qh[8], ql[8];
   float c_row;  // 2^-k: the power of two taken out of the row
+  uint32_t q_out;  // the wave's rows (bit n) that the split does not hold
   {
     const bool on = row < n_rows;
     const int q = on ? row / grp : 0, head = kvh * grp + (on ? row % grp : 0);
@@ -458,18 +507,24 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
         for (int i = 0; i < 4; ++i) x[b][i] = u[i], x[b][4 + i] = v[i];
       }
     }
-    float mx = 0.0f;
+    float mx = 0.0f, least = INFINITY;  // of the lane's 8-dim groups that are not zero, the least maximum
 #pragma unroll
-    for (int b = 0; b < 8; ++b)
+    for (int b = 0; b < 8; ++b) {
+      float mb = 0.0f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         x[b][i] *= sl2;
-        mx = fmaxf(mx, fabsf(x[b][i]));
+        mb = fmaxf(mb, fabsf(x[b][i]));
       }
+      mx = fmaxf(mx, mb);
+      if (mb > 0.0f) least = fminf(least, mb);
+    }
     mx = max_groups4(mx);
+    const uint64_t far = __ballot(least < mx * 0x1p-10f || mx == INFINITY);
+    q_out = (uint32_t)(far | far >> 16 | far >> 32 | far >> 48) & 0xffffu;
     // exponent that brings mx to [2^8, 2^9); zero rows and infinities stay as they are
     const int ex = (int)(__builtin_bit_cast(uint32_t, mx) >> 23) - 127;
-    const int k = (mx > 0.0f && ex < 128) ? max(-100, min(100, 8 - ex)) : 0;
+    const int k = (mx > 0.0f && ex < 128) ? min(126, 8 - ex) : 0;
     c_row = __builtin_ldexpf(1.0f, -k);
 #pragma unroll
     for (int b = 0; b < 8; ++b)
@@ -584,44 +639,56 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
           for (int i = 0; i < 4; ++i) s[kt][i] *= ks[i];
         }
       }
-      // K rows outside the products: their scores in f32 from the cache
+      // K rows outside the products (for queries outside them, all): their scores on
+      // the f32 matrix instruction, K from the cache and q as it came. Lane (n, g)
+      // brings dims 64 g .. 64 g + 63 of key n of a tile and of its row.
       const uint32_t out_keys = (uint32_t)__ballot(km_lane != 0);
-      if (out_keys) {
-        const int k_rb = (int)row_bytes(p.kt, kHD), k_stride = p.n_head_kv * k_rb;
-        auto load_k = [&](const uint8_t *kr, int d, float v[4]) RD4_INLINE {
-          if constexpr (KT >= 0) load4<KT>(kr, d, v);
-          else if constexpr (!KLO) load4<F16>(kr, d, v);
-          else if (p.kt == Q8_0) load4<Q8_0>(kr, d, v);
-          else if (p.kt == Q4_0) load4<Q4_0>(kr, d, v);
-          else if (p.kt == Q5_0) load4<Q5_0>(kr, d, v);
-          else load4<Q4_1>(kr, d, v);
-        };
-        int rr = min(row, n_rows - 1), gg = g;
-        __asm__ volatile("" : "+v"(rr), "+v"(gg));  // (addresses formed here, not held through the loop)
-        const int64_t qat = ((int64_t)(rr / grp) * p.n_head + kvh * grp + rr % grp) * kHD;
-        const float sl2 = p.scale * kLog2e, up = 1.0f / c_row;  // (up: a power of two)
+      if (out_keys | q_out) {
+        const PrefillArgs pa = args_again();
+        const uint8_t *pk = global_ptr(pa.k), *pq = global_ptr((const uint8_t *)pa.q);
+        const int k_rb = (int)row_bytes(pa.kt, kHD), k_stride = pa.n_head_kv * k_rb;
+        const int ga = pa.n_head / pa.n_head_kv;
+        int rr = min(row, pa.n_q * ga - 1), d0 = 64 * g;
+        __asm__ volatile("" : "+v"(rr), "+v"(d0));  // (addresses formed here, not held through the loop)
+        const int64_t qat = ((int64_t)(rr / ga) * pa.n_head + kvh * ga + rr % ga) * kHD + d0;
+        const float sl2 = pa.scale * kLog2e, up = 1.0f / c_row;  // (up: a power of two)
+        const uint32_t mine = ((q_out >> n) & 1 ? ~0u : out_keys) >> (4 * g);
 #pragma unroll 1
-        for (int key = 0; key < kBN; ++key) {
-          if (!((out_keys >> key) & 1) || j0 + key > kend) continue;  // (past kend a valid row was read again)
-          const uint8_t *kr = p.k + (int64_t)(j0 + key) * k_stride + (int64_t)kvh * k_rb;
-          float dot = 0.0f;
-#pragma unroll 1
-          for (int d0 = 0; d0 < kHD; d0 += 16) {
-            const int d = d0 + 4 * gg;
-            float kv[4], qv[4];
-            load_k(kr, d, kv);
-            if (p.q_f16) load4<F16>((const uint8_t *)p.q + 2 * qat, d, qv);
-            else load4<F32>((const uint8_t *)p.q + 4 * qat, d, qv);
+        for (int kt = 0; kt < 2; ++kt) {
+          if (!(q_out | ((out_keys >> (16 * kt)) & 0xffffu)) || j0 + 16 * kt > kend) continue;
+          // (keys past kend re-read a valid row: masked below)
+          const uint8_t *kr = pk + (int64_t)(j0 + min(16 * kt + n, kend - j0)) * k_stride + (int64_t)kvh * k_rb;
+          floatx4 f[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+          constexpr bool kTight = KLO && KT < 0;
+          auto block = [&](auto type, int h) RD4_INLINE {
+            RowBlock<decltype(type)::value> kb;
+            kb.read(kr, (d0 >> 5) + h);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) dot = fmaf(qv[c] * sl2 * up, kv[c], dot);
+            for (int c = 0; c < 8; ++c) {  // 4 dims at a time (few registers beside O and q)
+              float x[4], kv[4];
+              if (pa.q_f16) load4<F16>(pq + 2 * qat, 32 * h + 4 * c, x);
+              else load4<F32>(pq + 4 * qat, 32 * h + 4 * c, x);
+              kb.values(c, kv);
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                f[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[i], x[i] * sl2 * up, f[i & 1], 0, 0, 0);
+              if (kTight || (c & 1)) __builtin_amdgcn_sched_barrier(0);
+            }
+          };
+#pragma unroll 1
+          for (int h = 0; h < 2; ++h) {
+            if constexpr (KT >= 0) block(type_c<KT>{}, h);
+            else if constexpr (!KLO) block(type_c<F16>{}, h);
+            else if (pa.kt == Q8_0) block(type_c<Q8_0>{}, h);
+            else if (pa.kt == Q4_0) block(type_c<Q4_0>{}, h);
+            else if (pa.kt == Q5_0) block(type_c<Q5_0>{}, h);
+            else block(type_c<Q4_1>{}, h);
           }
-          dot += __shfl_xor(dot, 16, 64);
-          dot += __shfl_xor(dot, 32, 64);
 #pragma unroll
-          for (int kt = 0; kt < 2; ++kt)
+          for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              if (16 * kt + i == (key & 0x13) && g == ((key >> 2) & 3)) s[kt][i] = dot;
+              if (t == kt && ((mine >> (16 * t + i)) & 1)) s[t][i] = f[0][i] + f[1][i];
         }
       }
       if (j0 + kBN - 1 > wave_min_lim) {  // wave-uniform
@@ -705,12 +772,14 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     // What entered as zeros (f16 values that are not finite, blocks of a quantized
     // cache outside the scaled range) is added here, for the rows that attend the key.
     if (__any(nf_lane != 0)) {
-      const int v_rb = (int)row_bytes(p.vt, kHD), v_stride = p.n_head_kv * v_rb;
+      const PrefillArgs pa = args_again();
+      const uint8_t *pv = global_ptr(pa.v);
+      const int v_rb = (int)row_bytes(pa.vt, kHD), v_stride = pa.n_head_kv * v_rb;
       auto load_v = [&](const uint8_t *vr, int d, float v[4]) RD4_INLINE {
         if constexpr (VT >= 0) load4<VT>(vr, d, v);
         else if constexpr (VFULL) load4<Q4_1>(vr, d, v);
-        else if (p.vt == Q8_0) load4<Q8_0>(vr, d, v);
-        else if (p.vt == Q4_0) load4<Q4_0>(vr, d, v);
+        else if (pa.vt == Q8_0) load4<Q8_0>(vr, d, v);
+        else if (pa.vt == Q4_0) load4<Q4_0>(vr, d, v);
         else load4<Q5_0>(vr, d, v);
       };
 #pragma unroll 1
@@ -724,18 +793,24 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
           for (int i = 0; i < 4; ++i)
             if (16 * kt + i == (key & 0x13)) x = pf[kt][i];
         x = __builtin_ldexpf(__shfl(x, 4 * (key & 12) + n, 64), kPShift - e_o);
-        const uint8_t *vr = p.v + (int64_t)(j0 + key) * v_stride + (int64_t)kvh * v_rb;
+        const uint8_t *vr = pv + (int64_t)(j0 + key) * v_stride + (int64_t)kvh * v_rb;
         const bool on = j0 + key <= lim_row;
+        constexpr int kTiles = VT >= 0 || VFULL ? 4 : 2;  // (4 where the type is read at run time spills)
 #pragma unroll
-        for (int dt = 0; dt < 16; ++dt) {
-          if (!((blocks >> (dt >> 1)) & 1)) continue;  // (uniform)
+        for (int d4 = 0; d4 < 16; d4 += kTiles) {  // kTiles dim tiles' loads in flight together
+          if (!((blocks >> (d4 >> 1)) & (kTiles == 4 ? 3 : 1))) continue;  // (uniform)
           int g4 = 4 * g;
-          __asm__ volatile("" : "+v"(g4)::"memory");  // (one tile's addresses at a time: all together spill)
-          float v[4];
-          load_v(vr, 16 * dt + g4, v);
+          __asm__ volatile("" : "+v"(g4)::"memory");  // (addresses formed here, not held through the loop)
+          float v[kTiles][4];
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            if (on && (VLO || !(fabsf(v[c]) < INFINITY))) o[dt][c] = fmaf(x, v[c], o[dt][c]);
+          for (int i = 0; i < kTiles; ++i) load_v(vr, 16 * (d4 + i) + g4, v[i]);
+#pragma unroll
+          for (int i = 0; i < kTiles; ++i)
+            if (on && ((blocks >> ((d4 + i) >> 1)) & 1)) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c)
+                if (VLO || !(fabsf(v[i][c]) < INFINITY)) o[d4 + i][c] = fmaf(x, v[i][c], o[d4 + i][c]);
+            }
         }
       }
     }
@@ -746,35 +821,37 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   float Ls = l_run;
   Ls += __shfl_xor(Ls, 16, 64);
   Ls += __shfl_xor(Ls, 32, 64);
-  if (row >= n_rows) return;
-  const int q = row / grp, head = kvh * grp + row % grp;
+  const PrefillArgs pe = args_again();
+  const int ge = pe.n_head / pe.n_head_kv;
+  if (row >= pe.n_q * ge) return;
+  const int q = row / ge, head = kvh * ge + row % ge;
   const float o_pw2 = __builtin_ldexpf(1.0f, e_o - kPShift);
-  if (p.n_ksplit > 1) {
-    const int64_t nr = (int64_t)p.n_q * p.n_head, rr = (int64_t)ksp * nr + (int64_t)q * p.n_head + head;
-    float *rec = p.part + rr * kHD;
+  if (pe.n_ksplit > 1) {
+    const int64_t nr = (int64_t)pe.n_q * pe.n_head, rr = (int64_t)ksp * nr + (int64_t)q * pe.n_head + head;
+    float *rec = pe.part + rr * kHD;
 #pragma unroll
     for (int dt = 0; dt < 16; ++dt)
       if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[dt] * o_pw2;  // (l = 0: the merge drops the record)
-    if (g == 0) *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run, Ls);
+    if (g == 0) *(float2 *)(pe.part + (int64_t)pe.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run, Ls);
     return;
   }
   const float inv = (m_run == -INFINITY || !(Ls > 0.0f)) ? 0.0f : o_pw2 / Ls;
-  const int64_t ob = ((int64_t)q * p.n_head + head) * kHD;
+  const int64_t ob = ((int64_t)q * pe.n_head + head) * kHD;
 #pragma unroll
   for (int dt = 0; dt < 16; ++dt) {
     const int d = 16 * dt + 4 * g;
     float v[4] = {o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv};
-    if (p.gate) {
-      float4 gv = *(const float4 *)(p.gate + ob + d);
+    if (pe.gate) {
+      float4 gv = *(const float4 *)(pe.gate + ob + d);
       float gs[4] = {gv.x, gv.y, gv.z, gv.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         gs[i] = 1.0f / (1.0f + expf(-gs[i]));
         v[i] *= gs[i];
       }
-      *(float4 *)(p.gate + ob + d) = make_float4(gs[0], gs[1], gs[2], gs[3]);
+      *(float4 *)(pe.gate + ob + d) = make_float4(gs[0], gs[1], gs[2], gs[3]);
     }
-    *(float4 *)(p.out + ob + d) = make_float4(v[0], v[1], v[2], v[3]);
+    *(float4 *)(pe.out + ob + d) = make_float4(v[0], v[1], v[2], v[3]);
   }
 }
 

@@ -1,5 +1,5 @@
 """Prefill over quantized caches where values lie far apart: blocks of one V row,
-blocks of one K row, and values that are not finite. The path
+blocks of one K row, parts of one query, and values that are not finite. The path
 holds its operands as f16 pairs; what such a pair cannot hold takes an f32 path, so
 the results keep the tolerance of the path's other tests (3e-6, there derived), here
 for each 32-dim block of the output by itself, and are infinite or NaN where the
@@ -64,16 +64,17 @@ def test_v_blocks_far_apart(rd4, orc, dev, kt, vt, bits, how):
 
 @pytest.mark.parametrize("kt,vt", [(2, 2), (3, 3), (4, 5), (5, 1)])
 @pytest.mark.parametrize("bits", [15, 19, 23, 26])
-def test_k_blocks_far_apart(rd4, orc, dev, kt, vt, bits):
+@pytest.mark.parametrize("q_tiny", [False, True])
+def test_k_blocks_and_queries_far_apart(rd4, orc, dev, kt, vt, bits, q_tiny):
     """K's block 5 is 2^bits of the others; the queries are zero there (the scores
-    come from the small blocks alone)."""
+    come from the small blocks alone) or 2^-bits of their other values."""
     import torch
     pos0, nq = 90, 40
     n = pos0 + nq
     x = orc.randn(n * NKV * HD, 1).reshape(n, NKV, 8, 32) * np.float32(2000 * 2.0 ** -bits)
     x[:, :, 5] *= np.float32(2.0 ** bits)
     q = orc.randn(nq * NH * HD, 3).reshape(nq, NH, 8, 32) * np.float32(2.0 ** bits / 2000)
-    q[:, :, 5] = 0
+    q[:, :, 5] *= np.float32(2.0 ** -bits if q_tiny else 0)
     q = q.reshape(nq, NH, HD)
     k, v = orc.store_rows(kt, x.ravel()), orc.store_rows(vt, orc.randn(n * NKV * HD, 2))
     err = block_error(run(rd4, torch, dev, q, k, v, pos0, kt, vt), oracle(orc, q, k, v, pos0, kt, vt))
@@ -86,10 +87,10 @@ def like_valu(rd4, torch, dev, monkeypatch, q, k, v, pos0, kt, vt):
     got = run(rd4, torch, dev, q, k, v, pos0, kt, vt)
     monkeypatch.setenv("RD4_PREFILL_GENERIC", "1")
     want = run(rd4, torch, dev, q, k, v, pos0, kt, vt)
-    fin = np.isfinite(want)
-    assert np.array_equal(np.isfinite(got), fin)
-    assert np.array_equal(np.isnan(got), np.isnan(want))
-    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    fin, inf = np.isfinite(want), np.isinf(want)
+    assert np.argwhere(np.isfinite(got) != fin)[:5].tolist() == []
+    assert np.argwhere(np.isnan(got) != np.isnan(want))[:5].tolist() == []
+    assert (got[inf] == want[inf]).all()
     assert np.linalg.norm(got[fin] - want[fin]) <= 2 * REL * np.linalg.norm(want[fin])
     return want
 
@@ -119,6 +120,30 @@ def test_infinite_k(rd4, orc, dev, monkeypatch, kt, vt, sign):
             d[0] = np.copysign(np.inf, sign * float(d[0]))
     want = like_valu(rd4, torch, dev, monkeypatch, q, k, v, pos0, kt, vt)
     assert np.isfinite(want[:, 6 * h + 6:]).all() and (kt != 1 or np.isfinite(want).all() == (sign < 0))
+
+
+@pytest.mark.parametrize("kt,vt", [(2, 2), (1, 3)])
+def test_infinite_queries(rd4, orc, dev, monkeypatch, kt, vt):
+    """An infinite query value (scores of -inf and +inf, or of -inf alone) and queries
+    near f32's largest. A NaN query gives NaN (the VALU kernel counts a row without
+    any score as one without keys: 0), and leaves the others of its CTA alone."""
+    import torch
+    pos0, nq = 60, 40
+    n = pos0 + nq
+    x = orc.randn(n * NKV * HD, 1).reshape(n, NKV, HD)
+    x[:, 1, 9] = 0.3 + np.abs(x[:, 1, 9])  # dim 9 of kv head 1: above 0 in every key
+    k, v = orc.store_rows(kt, x.ravel()), orc.store_rows(vt, orc.randn(n * NKV * HD, 2))
+    q = orc.randn(nq * NH * HD, 3).reshape(nq, NH, HD)
+    q[3, 2, 40], q[9, 7, 9], q[17, 8, 9] = np.inf, -np.inf, np.inf
+    q[25] *= np.float32(2.0 ** 120)  # finite: one key has all the weight
+    like_valu(rd4, torch, dev, monkeypatch, q, k, v, pos0, kt, vt)
+    monkeypatch.delenv("RD4_PREFILL_GENERIC")
+    clean = run(rd4, torch, dev, q, k, v, pos0, kt, vt)
+    q[30, 20, 0] = np.nan
+    got = run(rd4, torch, dev, q, k, v, pos0, kt, vt)
+    assert np.isnan(got[30, 20]).all()
+    clean[30, 20] = got[30, 20]
+    assert np.array_equal(got, clean, equal_nan=True)
 
 
 @pytest.mark.parametrize("kt,vt", [(2, 2), (3, 3), (1, 5), (5, 4), (2, 1)])
