@@ -15,13 +15,13 @@
 //   * a quantized key row is scaled by a power of two (its largest block scale
 //     comes to [2^7, 2^8)) and split: d * int has at most 19 significant bits, so
 //     K' = kh + kl exactly (blocks down to 2^-21 of the row's largest scale);
-//   * S = kl.qh + kh.ql + kh.qh, f32 accumulation, then times both powers of two;
+//   * S = kl.qh + kh.ql + kh.qh (q4_1: + kl.ql), f32 accumulation, then times both powers of two;
 //     the scores of a key row that this does not hold (scales further apart, values
 //     that are not finite) are formed in f32 from the row itself;
 //   * value rows are scaled by a power of two 2^e of the CTA (its block of 32 keys
 //     has its largest block scale between 1 and 2^8; a block that has not moves e,
 //     and O with it) and split like keys, exactly for blocks down to 2^-14;
-//   * p stays f32 for the row sum l; p * 2^7 is split for O += vl.ph + vh.pl + vh.ph:
+//   * p stays f32 for the row sum l; p * 2^7 is split for O += vl.ph + vh.pl + vh.ph (q4_1: + vl.pl):
 //     22 bits of a p down to 2^-10 of the row's largest, below that 2^-32 of the
 //     largest;
 //   * V blocks that this does not hold (scales further apart, or not finite) enter
@@ -353,7 +353,9 @@ constexpr int kRing = 3;  // (2 to 5: within 1%)
 // KT, VT: the cache types, or -1 for a type read at run time. KLO, VLO: the rows
 // have remainder parts (all but f16); VFULL: q4_1 values, whose remainders are as
 // full as p's, take the fourth product vl.pl too (at 120 queries over 120 keys the
-// error is 1.04 times the VALU kernel's without it, 0.88 with).
+// error is 1.04 times the VALU kernel's without it, 0.88 with); q4_1 keys take
+// kl.ql likewise (1 query over 31 keys 1.23 times, 0.94 with it; 512 over 8192 385 us,
+// 414 with it).
 template <int T>
 using type_c = std::integral_constant<int, T>;
 template <int KT, int VT, bool KLO, bool VLO, bool VFULL>
@@ -463,8 +465,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     else switch (p.kt) {
       case Q8_0: convert_as(type_c<Q8_0>{}, std::false_type{}, st); break;
       case Q4_0: convert_as(type_c<Q4_0>{}, std::false_type{}, st); break;
-      case Q5_0: convert_as(type_c<Q5_0>{}, std::false_type{}, st); break;
-      default: convert_as(type_c<Q4_1>{}, std::false_type{}, st); break;
+      default: convert_as(type_c<Q5_0>{}, std::false_type{}, st); break;
     }
   };
   auto convert_v = [&](int st) RD4_INLINE {
@@ -618,7 +619,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
         if (KLO) sc[4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, fl[f % D]), qh[b], sc[4], 0, 0, 0);
         sc[b & 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[b], sc[b & 3], 0, 0, 0);
         sc[4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[b], sc[4], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        if (KT == Q4_1) sc[4] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, fl[f % D]), ql[b], sc[4], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         if (b == 7) s[kt] = ((sc[0] + sc[1]) + (sc[2] + sc[3])) + sc[4];
       }
@@ -681,8 +682,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
             else if constexpr (!KLO) block(type_c<F16>{}, h);
             else if (pa.kt == Q8_0) block(type_c<Q8_0>{}, h);
             else if (pa.kt == Q4_0) block(type_c<Q4_0>{}, h);
-            else if (pa.kt == Q5_0) block(type_c<Q5_0>{}, h);
-            else block(type_c<Q4_1>{}, h);
+            else block(type_c<Q5_0>{}, h);
           }
 #pragma unroll
           for (int t = 0; t < 2; ++t)
@@ -885,6 +885,8 @@ hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_
   else if (kt == Q5_0 && vt == Q5_0) launch<Q5_0, Q5_0>(q, grid, st);
   else if (kt == Q4_1 && vt == Q4_1) launch<Q4_1, Q4_1>(q, grid, st);
   else if (kt == Q5_0 && vt == Q4_1) launch<Q5_0, Q4_1>(q, grid, st);
+  else if (kt == Q4_1 && vt == F16) launch<Q4_1, F16>(q, grid, st);
+  else if (kt == Q4_1) launch<Q4_1, -1, true, true, false>(q, grid, st);
   else if (kt == F16 && vt == Q4_1) launch<F16, -1, false, true, true>(q, grid, st);
   else if (kt == F16) launch<F16, -1, false, true, false>(q, grid, st);
   else if (vt == F16) launch<-1, F16, true, false, false>(q, grid, st);

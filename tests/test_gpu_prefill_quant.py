@@ -148,3 +148,23 @@ def test_an_f16_v_value_that_is_not_finite_stays_with_its_readers(rd4, orc, dev)
     assert np.array_equal(got[~hit], clean[~hit])
     assert not np.isfinite(got[hit]).any()
     assert np.all(got[7:, 6 * h:6 * h + 6, 5] == np.inf)
+
+
+@pytest.mark.parametrize("vt", [1, 2, 5])
+def test_q4_1_keys_no_less_precise_than_valu_kernel(rd4, orc, dev, monkeypatch, vt):
+    """q4_1 K values fill both parts of their f16 pairs (d * q + m), so the product of
+    the two remainders counts: without it the error over these short contexts is 1.04
+    to 1.23 times the VALU kernel's, with it 0.88 to 0.96 (sums of five seeds' errors)."""
+    import torch
+    nh, nkv = 24, 4
+    for nq, pos0 in ((1, 30), (33, 0)):
+        err = {"0": 0.0, "1": 0.0}
+        for seed in range(5):
+            n = pos0 + nq
+            k, v = rows_of(orc, 5, n, nkv, 10 * seed + 1), rows_of(orc, vt, n, nkv, 10 * seed + 2)
+            q = orc.randn(nq * nh * 256, 10 * seed + 3).reshape(nq, nh, 256)
+            want = orc.attn_batch(q, k, v, pos0 + np.arange(nq, dtype=np.int32), nh, nkv, 256, 1 / 16, 5, vt, threads=8)
+            for env in err:
+                monkeypatch.setenv("RD4_PREFILL_GENERIC", env)
+                err[env] += rel(run(rd4, torch, dev, q, k, v, pos0, nh, nkv, 5, vt)[0], want)
+        assert err["0"] <= err["1"], (nq, pos0, err)
