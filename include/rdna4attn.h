@@ -57,7 +57,9 @@ const char *rd4_version(void);
  * on different streams never share records or counters; a stream's scratch is
  * created by its first split launch (hipMalloc plus a stream-ordered fill
  * kernel, no synchronisation) unless rd4_init / rd4_stream_init made it
- * first. Call them at init to keep allocation out of the first step. No
+ * first. Call them at init to keep allocation out of the first step. rd4_init
+ * also makes what streams without scratch take while they capture a graph: one
+ * spare set, and one spare buffer for the records of prefill calls. No
  * counterpart in the reference (its graph owned the partial buffer,
  * graph.cuh:771-778). */
 int rd4_init(void);

@@ -58,6 +58,10 @@ bool valid_type(int t) { return t >= 0 && t < kNumTypes; }
 // (no synchronisation), or, while it is capturing a HIP graph (when nothing may
 // be allocated), the spare. Sets are never freed. Caller-owned `partial` buffers are used instead when the
 // records fit (see run_attn).
+// Prefill's key splits need records alone, and run without them: a stream that has
+// no set gets a record buffer (the stream's set takes it over when one is made), a
+// capturing one rd4_init's spare record buffer. They never take the spare set, which
+// a decode captured later cannot do without.
 constexpr int64_t kPartialFloats = 16ll << 20;  // 64 MiB of records per stream
 constexpr int64_t kCounterWords = 1 << 20;
 struct Scratch {
@@ -67,24 +71,43 @@ struct Scratch {
 };
 std::map<std::pair<int, uintptr_t>, Scratch> g_scratch;
 std::map<int, std::vector<Scratch>> g_spare;  // per device, made by rd4_init, not yet assigned
+std::map<std::pair<int, uintptr_t>, float *> g_records;  // prefill's, of streams without a set
+std::map<int, std::vector<float *>> g_spare_records;
 std::mutex g_scratch_mu;
 
-// A new set on the current device; its counters are zeroed by a fill kernel on
-// `st` (waited for when `blocking`).
-int new_scratch(hipStream_t st, bool blocking, Scratch *out) {
+// kPartialFloats of records on the current device, or nullptr (the failed call's
+// error is not left for the next launch's check).
+float *new_records() {
+  float *p = nullptr;
+  if (hipMalloc(&p, kPartialFloats * sizeof(float)) == hipSuccess) return p;
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+// A new set on the current device, around `records` if there are any; its counters
+// are zeroed by a fill kernel on `st` (waited for when `blocking`).
+int new_scratch(hipStream_t st, bool blocking, float *records, Scratch *out) {
   Scratch n;
+  n.partial_c = records ? records : new_records();
   // Uncached: the generic kernel's split records cross XCDs inside one launch
   // (see merge.hpp). Uncached memory is never freed once a kernel has read it.
-  if (hipExtMallocWithFlags((void **)&n.partial, kPartialFloats * sizeof(float),
-                            hipDeviceMallocUncached) != hipSuccess ||
-      hipMalloc(&n.partial_c, kPartialFloats * sizeof(float)) != hipSuccess ||
-      hipMalloc(&n.counters, kCounterWords * sizeof(unsigned)) != hipSuccess)
+  if (!n.partial_c || hipMalloc(&n.counters, kCounterWords * sizeof(unsigned)) != hipSuccess ||
+      hipExtMallocWithFlags((void **)&n.partial, kPartialFloats * sizeof(float), hipDeviceMallocUncached) != hipSuccess) {
+    if (n.counters) (void)hipFree(n.counters);
+    if (!records && n.partial_c) (void)hipFree(n.partial_c);
+    (void)hipGetLastError();
     return fail(RD4_ENOMEM, "scratch allocation failed%s");
+  }
   const bool ok = fill_u32_launch(n.counters, kCounterWords, 0u, st) == hipSuccess &&
                   (!blocking || hipStreamSynchronize(st) == hipSuccess);
   if (!ok) return fail(RD4_ELAUNCH, "scratch counter fill failed%s");
   *out = n;
   return RD4_OK;
+}
+
+bool is_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  return st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
 int current_device(int *dev) {
@@ -99,11 +122,11 @@ int get_scratch(hipStream_t st, Scratch **out) {
   auto it = g_scratch.find({dev, (uintptr_t)st});
   if (it == g_scratch.end()) {
     Scratch n;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool capturing = st && hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
     std::vector<Scratch> &sp = g_spare[dev];
-    if (!capturing) {
-      if ((rc = new_scratch(st, false, &n))) return rc;
+    if (!is_capturing(st)) {
+      auto own = g_records.find({dev, (uintptr_t)st});
+      if ((rc = new_scratch(st, false, own == g_records.end() ? nullptr : own->second, &n))) return rc;
+      if (own != g_records.end()) g_records.erase(own);
     } else if (!sp.empty()) {  // nothing may be allocated while a graph is captured
       n = sp.back();
       sp.pop_back();
@@ -114,6 +137,28 @@ int get_scratch(hipStream_t st, Scratch **out) {
   }
   *out = &it->second;
   return RD4_OK;
+}
+
+// Records of a prefill call on `st` (kPartialFloats), or nullptr: the call runs
+// unsplit then.
+float *prefill_records(hipStream_t st) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return nullptr;
+  const std::pair<int, uintptr_t> key(dev, (uintptr_t)st);
+  std::lock_guard<std::mutex> lk(g_scratch_mu);
+  auto set = g_scratch.find(key);
+  if (set != g_scratch.end()) return set->second.partial_c;
+  auto own = g_records.find(key);
+  if (own != g_records.end()) return own->second;
+  float *p = nullptr;
+  if (!is_capturing(st)) {
+    p = new_records();
+  } else if (!g_spare_records[dev].empty()) {
+    p = g_spare_records[dev].back();
+    g_spare_records[dev].pop_back();
+  }
+  if (p) g_records.emplace(key, p);
+  return p;
 }
 
 int check_attn_shape(int n_head, int n_head_kv, int head_dim, int kt, int vt) {
@@ -329,20 +374,26 @@ const char *rd4_version(void) { return "rdna4attn-gfx950 0.1"; }
 int rd4_init(void) {
   int dev = 0, rc;
   if ((rc = current_device(&dev))) return rc;
-  // The null stream's set, and one spare for the next stream seen (a graph
-  // capture stream included), zeroed with a blocking memset: this is the init
-  // call, not a launch.
+  // The null stream's set, and one spare set and one spare record buffer for the
+  // next streams that capture a graph, the counters zeroed and waited for: this is
+  // the init call, not a launch.
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   if (!g_scratch.count({dev, (uintptr_t)0})) {
     Scratch n;
-    if ((rc = new_scratch(nullptr, true, &n))) return rc;
+    if ((rc = new_scratch(nullptr, true, nullptr, &n))) return rc;
     g_scratch.emplace(std::make_pair(dev, (uintptr_t)0), n);
   }
   std::vector<Scratch> &sp = g_spare[dev];
   if (sp.empty()) {
     Scratch n;
-    if ((rc = new_scratch(nullptr, true, &n))) return rc;
+    if ((rc = new_scratch(nullptr, true, nullptr, &n))) return rc;
     sp.push_back(n);
+  }
+  std::vector<float *> &sr = g_spare_records[dev];
+  if (sr.empty()) {
+    float *p = new_records();
+    if (!p) return fail(RD4_ENOMEM, "scratch allocation failed%s");
+    sr.push_back(p);
   }
   FixedScratch f;
   if ((rc = fixed_scratch(&f))) return rc;
@@ -553,17 +604,8 @@ void prefill_part(PrefillArgs &p, int kt, int vt, hipStream_t st) {
     return;
   const int s = prefill_ksplits(p, kt, vt, kPartialFloats);
   if (s <= 1 || prefill_part_floats(p, s) > kPartialFloats) return;
-  // a stream without a set under graph capture runs unsplit: the lookup's
-  // failure is not the call's, so its message is not left behind
-  char saved[sizeof(g_err)];
-  std::memcpy(saved, g_err, sizeof(g_err));
-  Scratch *sc = nullptr;
-  if (get_scratch(st, &sc) == RD4_OK) {
-    p.part = sc->partial_c;
-    p.part_floats = kPartialFloats;
-  } else {
-    std::memcpy(g_err, saved, sizeof(g_err));
-  }
+  p.part = prefill_records(st);
+  if (p.part) p.part_floats = kPartialFloats;
 }
 
 int rd4_fa2_prefill_usable(int kt, int vt, int n_q, int pos0, int n_head, int n_head_kv,
