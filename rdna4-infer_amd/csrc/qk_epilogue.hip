@@ -202,9 +202,11 @@ __global__ __launch_bounds__(64 * kEpiWaves) void qk_epilogue_kernel(EpiArgs a) 
 
       if (a.n_rot > 0) {
         float *row = rows[wave];
-        // the row is exchanged between the lanes of this wave only (the first
-        // fence orders it behind the previous row's reads)
+        // the row is exchanged between the lanes of this wave only: its writes stay
+        // behind the reads of the wave's previous row, its reads behind them
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (on) {
 #pragma unroll
           for (int g = 0; g < G; ++g)
