@@ -221,7 +221,7 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
   // (and with three waves per SIMD the registers allow shorter rings only)
   constexpr int kQD = NSL > 1 ? 2 : W > 8 ? RD4_PF_QKD_W12 : kQD0;
   constexpr int kPVD = NSL > 1 ? 2 : W > 8 ? RD4_PF_PVD_W12 : kPVD0;
-  extern __shared__ __align__(16) uint8_t smem[];
+  extern __shared__ __align__(512) uint8_t smem[];  // (512: the operand addresses XOR the low bits)
   // the wave index is uniform: readfirstlane keeps DMA bases and LDS
   // destinations in scalar registers
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;

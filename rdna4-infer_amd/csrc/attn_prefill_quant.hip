@@ -200,13 +200,11 @@ __device__ __forceinline__ void split_mul_add(half2v q, half2v d, half2v m, uint
   lo = as_u32(err + l);
 }
 
-// Convert one 32-value block of type T, its bytes in LDS at row + b * block
-// bytes (row 4-byte aligned; blocks start 2 bytes off a word where b is odd
-// except q4_1's), into 16 hi words and 16 lo words (f16 pairs of consecutive
-// elements). pw2 is the power of two that the row's values are scaled by.
+// The words of 32-value block b of a row (4-byte aligned; blocks start 2 bytes off a
+// word where b is odd, except q4_1's): *dm its scale d (q4_1: d | offset m << 16), w
+// the data behind it (q5_0: the high bits, then the nibbles; q4_1: the nibbles).
 template <int T>
 __device__ __forceinline__ void block_words(const uint8_t *row, int b, uint32_t *w, uint32_t *dm) {
-  // w: the block's data words after d (q5_0: the high bits, then the nibbles; q4_1: nibbles), dm: d | m << 16
   constexpr int BB = block_bytes(T);
   constexpr int NW = T == Q8_0 ? 8 : T == Q5_0 ? 5 : 4;
   const uint32_t *p = (const uint32_t *)(row + ((BB * b) & ~3));
@@ -361,7 +359,7 @@ using type_c = std::integral_constant<int, T>;
 template <int KT, int VT, bool KLO, bool VLO, bool VFULL>
 __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p) {
   using L = Lds<KLO, VLO>;
-  extern __shared__ __align__(16) uint8_t smem[];
+  extern __shared__ __align__(512) uint8_t smem[];  // (512: the operand addresses XOR the low bits)
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int n = lane & 15, g = lane >> 4;
   const int grp = p.n_head / p.n_head_kv;
@@ -385,7 +383,7 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
   auto limit_of = [&](int row) RD4_INLINE -> int {
     if (row >= n_rows) return -1;
     const int q = row / grp;
-    return min(p.pos ? p.pos[q] : p.pos0 + q, p.kmax);
+    return min(p.pos0 + q, p.kmax);
   };
   int kend;  // last key that any row of the CTA attends
   {

@@ -116,7 +116,9 @@ hipError_t prefill_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st) 
   // kernel's is shorter: 16 queries over 16 q8_0 keys 17.2 us there, 18.9 us on
   // the matrix cores; 64 over 64 30.8 against 24.1 us, 512 over 8192 6121
   // against 350 us.
-  if ((al & 15) == 0 && p.kmax >= 24 && prefill_quant_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim))
+  // (That kernel knows consecutive positions only; no entry point passes others
+  // with a quantized cache.)
+  if ((al & 15) == 0 && !p.pos && p.kmax >= 24 && prefill_quant_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim))
     return prefill_quant_launch(kt, vt, p, st);
   AttnArgs a{};
   a.q = (const float *)p.q;
