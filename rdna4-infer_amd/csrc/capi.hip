@@ -174,7 +174,7 @@ int check_attn_shape(int n_head, int n_head_kv, int head_dim, int kt, int vt) {
 // (the MFMA kernel's CTA fills a CU; the generic kernel's takes a quarter of
 // one), and at least `min_keys` keys per split. CTAs that fill a CU run in
 // rounds, so their count stays at or below the target: one CTA more is a second
-// round (5 tokens at 4000 f16 keys: 22 splits in 264 CTAs 22.9 us, 21 in 252 17.2
+// round (5 tokens at 4000 f16 keys: 22 splits in 264 CTAs 21.1 us, 21 in 252 15.6
 // us per layer).
 int auto_splits(int keys, int ctas_per_split, int target, int min_keys, bool fills_cu) {
   static const int env = [] {  // tuning override, read once

@@ -30,8 +30,10 @@ int compute_units() {
 // Rows per CTA and keys per block of a cache pair's MFMA kernel, and what a CTA
 // costs on an MI355X: us per key block, and us before and after its blocks. (The
 // f16 kernel's blocks take 2.2 us in a long call on few CUs and 3.2 on all; with a
-// few blocks each, first use and masks included, 3.4, and that is where the count
-// is close: 168 queries from position 0 take 32.1 us in one split, 26.9 in three.)
+// few blocks each, first use and masks included, 3.4. The last is taken for all calls:
+// it decides where the counts are close, 168 gated queries from position 0 (32.1 us
+// in one split, 26.9 in three), and a long call's best count differs little from its
+// neighbours.)
 struct Shape {
   int rows, keys;
   double block_us, cta_us;
@@ -50,13 +52,20 @@ constexpr double kMergeUs = 2.0, kMergeBytesPerUs = 5e6;
 // estimated time: the CTAs of one round all run at once; a further round costs a
 // whole CTA when the rows see about the same keys (a long prefix), and less when
 // they differ (causal rows from position 0, heaviest first); the merge costs its
-// launch and the records' traffic. Measured over split counts 1 to 64 (us: one
-// split / the count taken): f16 201 queries over 1534 keys 76 / 38, 64 over 8064
-// 282 / 42, 16 over 30016 992 / 45, 512 over 8192 288 / 126, 512 over 512 44 /
-// 38, 1000 over 2000 96 / 79; q8_0 16 over 8016 855 / 39, 64 over 1064 126 / 30,
-// 512 over 8192 852 / 350, 512 over 512 74 / 50. The count taken is within 5% of
-// the best in 20 of 24 such calls and within 16% in the others but one (q8_0, 64
-// queries over 8064 keys, whose best count is not a divisor).
+// launch and the records' traffic. Measured with these constants, calls in a row on one
+// cache, no gate, merge included, forced counts of 1 to 64 beside the one taken (us: one split
+// / best forced / taken). f16: 201 queries over 1534 keys 63 / 34 / 34, 64 over 8064
+// 262 / 38 / 39, 16 over 30016 943 / 43 / 42, 512 over 8192 268 / 123 / 116, 512 over
+// 512 32 / 31 / 34, 1000 over 2000 83 / 68 / 68, 168 over 168 21 / 21 / 23, 97 over 397
+// 28 / 25 / 26, 700 over 700 39 / 37 / 39; q8_0: 16 over 8016 733 / 37 / 37, 64 over
+// 1064 108 / 31 / 31, 512 over 8192 741 / 353 / 343, 512 over 512 58 / 42 / 46, 64 over
+// 8064 734 / 64 / 60, 700 over 700 78 / 60 / 77, 900 over 4900 455 / 364 / 455. Over 26
+// calls the count taken is within 5% of the best in 20, within 11% in four more; the
+// last two of the list (q8_0, a second round of CTAs that costs less than the estimate)
+// are 27 and 25% off. These calls have no gate. With one, which an unsplit CTA applies
+// at its end and the merge launch in many more waves, short calls gain most: 168 over
+// 168 with its gate and stores 42 us in one split, 31 in the count taken, 512 over 512
+// 57 and 46; the f16 constants are theirs.
 // RD4_PREFILL_KSPLIT forces a count (1: never split).
 int prefill_ksplits(const PrefillArgs &p, int kt, int vt, int64_t max_floats) {
   static const int env = [] {
