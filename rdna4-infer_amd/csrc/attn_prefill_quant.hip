@@ -6,7 +6,7 @@
 // i at position p_i attends keys 0..min(p_i, kmax), dequantized as kv_load<>
 // (kv.h:174-368), f32 softmax and accumulation, then the optional sigmoid gate.
 //
-// Precision: f32 sums, and an error at or below that of f32 operands, on f16 matrix
+// Precision: f32 sums, and the error of f32 operands or less, on f16 matrix
 // instructions. Every operand enters as an f16 hi part plus the f16 remainder (22
 // bits where f32 has 24):
 //   * a query row is scaled by a power of two (its largest |q * scale * log2e|
@@ -30,10 +30,13 @@
 // f16 rows have no remainder part (and no scaling): two products instead of three.
 // Relative error against 64 bits, the VALU kernel (attn_generic.hip), which took
 // these calls before, in brackets, for q8_0: 1.2e-7 (1.3e-7) at 33 queries over 33
-// keys, 2.1e-7 (2.6e-7) over 233, 3.5e-7 (8.8e-7) over 8064. What it takes: the
+// keys, 2.1e-7 (2.6e-7) over 233, 3.5e-7 (8.8e-7) over 8064; 0.23 to 0.98 times that
+// kernel's in 300 calls of 25 to 2300 queries over up to 32768 keys, queries and caches
+// near N(0, 1). (Queries of 0.2 over 28 to 100 q8_0 or q4_0 keys: 1.03 to 1.07, where
+// vl.pl, left out, shows beside few other roundings.) What it takes: the
 // large products of S in four sums and the small ones in a fifth (one sum for
-// all: 2.0 times the error at 233 keys), and the p split near 2^7 (near 1: 1.5
-// times). V's power of two is no part of p (a row's own exponent in p, as 2^e of it:
+// all: 2.0 times the error at 233 keys), the p split near 2^7 (near 1: 1.5
+// times), and O rounded once per block where a CTA sums most of a row (BSUM below). V's power of two is no part of p (a row's own exponent in p, as 2^e of it:
 // rows 2^17 smaller than another lost percents of what they add where the other's
 // dims are zero).
 //
@@ -354,10 +357,16 @@ constexpr int kRing = 3;  // (2 to 5: within 1%)
 // full as p's, take the fourth product vl.pl too (at 120 queries over 120 keys the
 // error is 1.04 times the VALU kernel's without it, 0.88 with); q4_1 keys take
 // kl.ql likewise (1 query over 31 keys 1.23 times, 0.94 with it; 512 over 8192 385 us,
-// 414 with it).
+// 414 with it). BSUM: a block's products with V are summed from zero and added to O once,
+// one tile behind, so that O is rounded once per block and not at each product: 64 adds
+// per block that no product hides. For calls of one or two splits, whose CTAs sum half of
+// a row's keys or more: 990 q4_0 queries over 4051 keys have 1.19 times the VALU
+// kernel's error without it, 0.56 with (374 us, 399 with it), rows 780 to 827 of 1660
+// from position 0 (two splits, theirs the first) 1.14 and 0.79 (103, 108 us). Shorter sums stay below that kernel's without it
+// (512 over 8192 in five splits: 0.6 times; 345 us, 365 with it).
 template <int T>
 using type_c = std::integral_constant<int, T>;
-template <int KT, int VT, bool KLO, bool VLO, bool VFULL>
+template <int KT, int VT, bool KLO, bool VLO, bool VFULL, bool BSUM>
 __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p) {
   using L = Lds<KLO, VLO>;
   extern __shared__ __align__(512) uint8_t smem[];  // (512: the operand addresses XOR the low bits)
@@ -755,15 +764,25 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
       };
 #pragma unroll
       for (int t = 0; t < D - 1; ++t) read_v(t);
+      floatx4 c;
+      auto add = [&](int t) RD4_INLINE {
+        o[t] += c;
+        __asm__ volatile("" : "+v"(o[t]));  // (here: moved to the block's end the sums spill)
+      };
 #pragma unroll
       for (int t = 0; t < 16; ++t) {
         if (t + D - 1 < 16) read_v(t + D - 1);
-        if (VFULL) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[t % D], pl, o[t], 0, 0, 0);
-        if (VLO) o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[t % D], ph, o[t], 0, 0, 0);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[t % D], pl, o[t], 0, 0, 0);
-        o[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[t % D], ph, o[t], 0, 0, 0);
+        floatx4 x = BSUM ? floatx4{0.f, 0.f, 0.f, 0.f} : o[t];
+        if (VFULL) x = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[t % D], pl, x, 0, 0, 0);
+        if (VLO) x = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl[t % D], ph, x, 0, 0, 0);
+        x = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[t % D], pl, x, 0, 0, 0);
+        x = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh[t % D], ph, x, 0, 0, 0);
+        if (BSUM && t > 0) add(t - 1);
+        if (BSUM) c = x;
+        else o[t] = x;
         __builtin_amdgcn_sched_barrier(0);
       }
+      if (BSUM) add(15);
     }
     if (more && isv) {
       landed();
@@ -869,7 +888,10 @@ bool prefill_quant_supported(int kt, int vt, int n_head, int n_head_kv, int head
 template <int KT, int VT, bool KLO = KT != F16, bool VLO = VT != F16, bool VFULL = VT == Q4_1>
 static void launch(const PrefillArgs &q, dim3 grid, hipStream_t st) {
   constexpr size_t lds = Lds<KLO, VLO>::kBytes;
-  hipLaunchKernelGGL((prefill_quant_kernel<KT, VT, KLO, VLO, VFULL>), grid, dim3(64 * kW), lds, st, q);
+  if (q.n_ksplit <= 2)
+    hipLaunchKernelGGL((prefill_quant_kernel<KT, VT, KLO, VLO, VFULL, true>), grid, dim3(64 * kW), lds, st, q);
+  else
+    hipLaunchKernelGGL((prefill_quant_kernel<KT, VT, KLO, VLO, VFULL, false>), grid, dim3(64 * kW), lds, st, q);
 }
 
 hipError_t prefill_quant_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st) {

@@ -57,12 +57,12 @@ constexpr double kMergeUs = 2.0, kMergeBytesPerUs = 5e6;
 // / best forced / taken). f16: 201 queries over 1534 keys 63 / 34 / 34, 64 over 8064
 // 262 / 38 / 39, 16 over 30016 943 / 43 / 42, 512 over 8192 268 / 123 / 116, 512 over
 // 512 32 / 31 / 34, 1000 over 2000 83 / 68 / 68, 168 over 168 21 / 21 / 23, 97 over 397
-// 28 / 25 / 26, 700 over 700 39 / 37 / 39; q8_0: 16 over 8016 733 / 37 / 37, 64 over
-// 1064 108 / 31 / 31, 512 over 8192 741 / 353 / 343, 512 over 512 58 / 42 / 46, 64 over
-// 8064 734 / 64 / 60, 700 over 700 78 / 60 / 77, 900 over 4900 455 / 364 / 455. Over 26
-// calls the count taken is within 5% of the best in 20, within 11% in four more; the
+// 28 / 25 / 26, 700 over 700 39 / 37 / 39; q8_0: 16 over 8016 777 / 37 / 37, 64 over
+// 1064 114 / 31 / 31, 512 over 8192 788 / 353 / 341, 512 over 512 62 / 42 / 48, 64 over
+// 8064 779 / 64 / 59, 700 over 700 81 / 61 / 76, 900 over 4900 482 / 354 / 482. Over 26
+// calls the count taken is within 5% of the best in 20, within 13% in four more; the
 // last two of the list (q8_0, a second round of CTAs that costs less than the estimate)
-// are 27 and 25% off. These calls have no gate. With one, which an unsplit CTA applies
+// are 25 and 36% off. These calls have no gate. With one, which an unsplit CTA applies
 // at its end and the merge launch in many more waves, short calls gain most: 168 over
 // 168 with its gate and stores 42 us in one split, 31 in the count taken, 512 over 512
 // 57 and 46; the f16 constants are theirs.
@@ -124,7 +124,7 @@ hipError_t prefill_launch(int kt, int vt, const PrefillArgs &p, hipStream_t st) 
   // A call with few keys is all launch and first-use latency, and the VALU
   // kernel's is shorter: 16 queries over 16 q8_0 keys 17.2 us there, 18.9 us on
   // the matrix cores; 64 over 64 30.8 against 24.1 us, 512 over 8192 6121
-  // against 350 us.
+  // against 341 us.
   // (That kernel knows consecutive positions only; no entry point passes others
   // with a quantized cache.)
   if ((al & 15) == 0 && !p.pos && p.kmax >= 24 && prefill_quant_supported(kt, vt, p.n_head, p.n_head_kv, p.head_dim))

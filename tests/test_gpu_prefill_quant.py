@@ -1,8 +1,8 @@
 """Prefill over quantized caches on the matrix cores against the f64 oracle and
 against the VALU kernel, at the edges of its tiles (128 rows per CTA, 32-key
 blocks), with and without key splits, and over value ranges that f16 cannot hold
-unscaled. The path computes in 32 bits (operands split into f16 pairs, 2^-22
-relative; f32 sums and probabilities), so the tolerance is that of f32 sums:
+unscaled. The path holds its operands as pairs of f16 values (2^-22 relative) and
+sums in f32, so the tolerance is that of f32 sums:
 relative error (2-norm) 3e-6 = 2^-22 for each of q, K and p * V added up, plus the
 roundings of sums over at most a few thousand terms (2^-24 sqrt(4000) = 4e-6 of a
 single term, averaged over the row's independent dims)."""
@@ -168,3 +168,22 @@ def test_q4_1_keys_no_less_precise_than_valu_kernel(rd4, orc, dev, monkeypatch, 
                 monkeypatch.setenv("RD4_PREFILL_GENERIC", env)
                 err[env] += rel(run(rd4, torch, dev, q, k, v, pos0, nh, nkv, 5, vt)[0], want)
         assert err["0"] <= err["1"], (nq, pos0, err)
+
+
+@pytest.mark.parametrize("kt,vt,nh,nkv,pos0,nq,r0", [(3, 3, 24, 4, 3061, 990, 942), (2, 2, 32, 8, 2300, 855, 807),
+                                                     (4, 5, 24, 4, 281, 941, 893), (3, 3, 16, 2, 0, 1660, 780)])
+def test_long_sums_no_less_precise_than_valu_kernel(rd4, orc, dev, monkeypatch, kt, vt, nh, nkv, pos0, nq, r0):
+    """Calls whose CTAs each sum all of a row's keys (row blocks enough for the GPU: one
+    split; the last case: two, and rows that end in the first): 48 rows from r0 on. With
+    O rounded at every product the error is 1.06 to 1.19 times the VALU kernel's, with one
+    rounding per key block 0.51 to 0.79."""
+    import torch
+    n = pos0 + nq
+    k, v = rows_of(orc, kt, n, nkv, 1), rows_of(orc, vt, n, nkv, 2)
+    q, rows = orc.randn(nq * nh * 256, 3).reshape(nq, nh, 256), slice(r0, r0 + 48)
+    pos = pos0 + np.arange(nq, dtype=np.int32)
+    want = orc.attn_batch(q[rows], k, v, pos[rows], nh, nkv, 256, 1 / 16, kt, vt, threads=8)
+    a = run(rd4, torch, dev, q, k, v, pos0, nh, nkv, kt, vt)[0][rows]
+    monkeypatch.setenv("RD4_PREFILL_GENERIC", "1")
+    b = run(rd4, torch, dev, q, k, v, pos0, nh, nkv, kt, vt)[0][rows]
+    assert rel(a, want) <= rel(b, want), (rel(a, want), rel(b, want))
