@@ -639,8 +639,9 @@ __global__ __launch_bounds__(64 * W, 1) void prefill_mfma_kernel(PrefillArgs p) 
       float *rec = p.part + rr * kHD;
 #pragma unroll
       for (int dt = 0; dt < 16; ++dt)
-        if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[sl][dt];  // (l = 0: the merge drops the record)
-      if (g == 0) *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run[sl], L);
+        if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[sl][dt];  // (the merge drops the record of an empty split)
+      if (g == 0)  // (l = -1: the row attends no key of the split)
+        *(float2 *)(p.part + (int64_t)p.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run[sl], lim_row[sl] < b0 * kBN ? -1.0f : L);
       continue;
     }
     const float inv = (m_run[sl] == -INFINITY || !(L > 0.0f)) ? 0.0f : 1.0f / L;
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs p) {
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= nr) return;
   const int S = p.n_ksplit;
-  float2 r = make_float2(-INFINITY, 0.0f);
+  float2 r = make_float2(-INFINITY, -1.0f);
   if (lane < S) r = *(const float2 *)(p.part + (int64_t)S * nr * kHD + 2 * (lane * nr + row));
   const float *rec = p.part + row * kHD + 4 * lane;
   constexpr int kB = 8;
@@ -688,12 +689,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs p) {
       if (s0 + i < S) rv[i] = *(const floatx4 *)(rec + (int64_t)(s0 + i) * nr * kHD);
   };
   load(0);
-  // A split with no key of this row has l = 0 and counts for nothing, whatever its
-  // record holds. m = -inf alone does not say so: where every score of a split is
-  // NaN the running max stays at -inf and l is NaN, and the row must end as NaN.
-  const bool empty = r.y == 0.0f;
+  // A split with no key of this row has l = -1 and counts for nothing, whatever its
+  // record holds. Neither m = -inf nor l = 0 says so: where every score of a split is
+  // NaN, m stays -inf and l is NaN; where every score is -inf, l is 0, and O is NaN in
+  // the dims of a V value that is not finite. Both reach the row with a weight of 0.
+  const bool empty = r.y < 0.0f;
   const float M = wave_max(r.x);
-  const float wgt = empty ? 0.0f : __builtin_amdgcn_exp2f(r.x - M);
+  const float wgt = r.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(r.x - M);
   const float L = wave_sum(empty ? 0.0f : wgt * r.y);
   const uint64_t used = ~__ballot(empty);
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};

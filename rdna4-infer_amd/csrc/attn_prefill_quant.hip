@@ -853,8 +853,9 @@ __global__ __launch_bounds__(64 * kW, 1) void prefill_quant_kernel(PrefillArgs p
     float *rec = pe.part + rr * kHD;
 #pragma unroll
     for (int dt = 0; dt < 16; ++dt)
-      if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[dt] * o_pw2;  // (l = 0: the merge drops the record)
-    if (g == 0) *(float2 *)(pe.part + (int64_t)pe.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run, Ls);
+      if (nbk > 0) *(floatx4 *)(rec + 16 * dt + 4 * g) = o[dt] * o_pw2;  // (the merge drops the record of an empty split)
+    if (g == 0)  // (l = -1: the row attends no key of the split)
+      *(float2 *)(pe.part + (int64_t)pe.n_ksplit * nr * kHD + 2 * rr) = make_float2(m_run, lim_row < b0 * kBN ? -1.0f : Ls);
     return;
   }
   const float inv = (m_run == -INFINITY || !(Ls > 0.0f)) ? 0.0f : o_pw2 / Ls;

@@ -61,3 +61,41 @@ def test_a_split_whose_scores_are_all_nan_stays_nan(rd4, orc, dev, kt, vt):
         hit[bad - pos0:, 6 * h:6 * h + 6] = True
         assert np.isnan(got[hit]).all(), bad
         assert np.array_equal(got[~hit], clean[~hit]), bad
+
+
+@pytest.mark.parametrize("kt,vt", [(1, 1), (2, 2), (4, 5), (1, 2), (3, 1)])
+def test_a_split_whose_scores_are_all_minus_infinity_keeps_its_v(rd4, orc, dev, kt, vt):
+    """One key whose scores are -inf and whose V is infinite, the first of a split: the
+    query at its position attends no other key of the split. Its weight is 0, and
+    0 * inf is NaN in V's dims, as where the key stands inside a split; the other dims
+    are those of the key left out."""
+    import torch
+    nh, nkv, pos0, nq, h, b = 24, 4, 400, 60, 1, 2
+    n = pos0 + nq
+    x = orc.randn(n * nkv * 256, 1).reshape(n, nkv, 256)
+    x[:, :, 64:96] = 0.5 + np.abs(x[:, :, 64:96])
+    q = orc.randn(nq * nh * 256, 3).reshape(nq, nh, 256)
+    q[:, :, 64:96] = 0.1 + np.abs(q[:, :, 64:96])
+    k, v = orc.store_rows(kt, x.ravel()), orc.store_rows(vt, orc.randn(n * nkv * 256, 2))
+    q = to_dev(q, torch, dev)
+
+    def run(kb, vb):
+        out = torch.zeros(q.shape, dtype=torch.float32, device=dev)
+        rd4.prefill(q, to_dev(kb, torch, dev), to_dev(vb, torch, dev), out, pos0, nh, nkv, 256, 1 / 16, kt, vt)
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    for bad in (447, 448):  # inside a split; the first key of one (of 32 and of 64 keys)
+        kb, vb = k.copy(), v.copy()
+        krow = kb.view(np.uint8).reshape(n, nkv, -1)[bad, h]
+        d = krow.view(np.float16)[70:71] if kt == 1 else krow.reshape(8, -1)[b, :2].view(np.float16)
+        d[0] = -np.inf if kt == 1 else np.copysign(np.inf, -float(d[0]))
+        left_out = run(kb, v)
+        vrow = vb.view(np.uint8).reshape(n, nkv, -1)[bad, h].reshape(8, -1)[b]
+        vrow[:2].view(np.float16)[0] = np.inf
+        got, dims = run(kb, vb)[bad - pos0, 6 * h:6 * h + 6], slice(32 * b, 32 * b + (1 if vt == 1 else 32))
+        want = left_out[bad - pos0, 6 * h:6 * h + 6]
+        assert np.isfinite(want).all(), bad
+        assert np.isnan(got[:, dims]).all(), bad
+        want[:, dims] = got[:, dims]
+        assert np.array_equal(got, want, equal_nan=True), bad
